@@ -335,7 +335,27 @@ struct FfnPlan {
     bool skinny13 = false;  // w1/w3 on the grouped skinny kernel (choose_skinny)
     bool skinny2 = false;   // w2 on it
     int w13_splits = 1;     // K splits of the skinny w1/w3 (their raw sums in sk_part)
+    bool fp32 = false;      // the tiles on fp32 MFMA (GemmArgs::fp32, few_rows)
 };
+
+// Layers whose experts hold few rows, at most 4 on average, or 16 with up to
+// 16 experts: they are bound by reading the weights, and the fp32 MFMA tiles,
+// whose loads run two K steps ahead, read them faster than the bf16 pieces,
+// whose loads run one ahead (same box, us, w1/w3 and w2: config 3 at 4 / 24
+// / 64 tokens fp32 566 / 938 / 924 and 280 / 413 / 435, pieces 750 / 1,003 /
+// 1,024 and 379 / 562 / 568; at 128 tokens, 32 rows each, 1,219 and 757
+// against 1,076 and 591.  Config 4's 64 experts, unevenly loaded, at 16 / 32
+// tokens 170 / 210 against 200 / 241; at 64 / 128 tokens, 8 and 16 rows each,
+// 342 / 395 against 275 / 304).
+bool few_rows(int64_t pairs, int64_t E) { return pairs <= 4 * E || (E <= 16 && pairs <= 16 * E); }
+
+int grouped_slots(moe_ctx* ctx, moe::GemmUse use, bool fp32, bool sk) {
+    int& occ = (sk ? ctx->sk_blocks_per_cu : ctx->grouped_blocks_per_cu)[fp32 ? 1 : 0]
+                                                                        [static_cast<int>(use)];
+    if (occ == 0)
+        occ = sk ? moe::gemm_sk_blocks_per_cu(use, fp32) : moe::gemm_blocks_per_cu(use, fp32);
+    return ctx->cus * occ;
+}
 
 // The K splits of w2 on one w2 tile and their modelled time (choose_w2_split_plan).
 struct W2SplitPlan {
@@ -344,7 +364,7 @@ struct W2SplitPlan {
 };
 
 W2SplitPlan choose_w2_split_plan(moe_ctx* ctx, int64_t pairs, int64_t d, int64_t d_ff, int64_t E,
-                                 int w2_tile);
+                                 int w2_tile, bool fp32);
 
 // The w1/w3 tile: 128 rows x 128 columns of each operand, or, when d_ff is
 // a multiple of 64 but not of 128 (the reference's 448), 256 rows x 64
@@ -392,17 +412,26 @@ int64_t expected_m_tiles(int64_t pairs, int64_t E, int bm) {
 // moe_ctx_set_stream_k) forces either (1: on every launch the direct
 // buffer-load path applies to, on all slots).  Returns the stream-K grid, 0
 // for one tile per workgroup.
+//
+// The bf16 pieces do the same work in half the time, so reading a tile's
+// operands alone, out of step with the tiles that share them, costs them more:
+// w1/w3 run stream-K only while the tiles fill at most 0.7 of the slots (us,
+// one tile per workgroup / stream-K: the reference's layer at 256 / 1,024 /
+// 4,096 tokens, fill 0.1 / 0.2 / 0.5, 387 / 405 / 548 against 120 / 170 / 454;
+// config 5 at 256 tokens, 0.3, 108 against 98; at 1,024, 0.9, 184 against 211;
+// config 3 at 256 / 4,096 tokens 1,210 / 11,101 against 1,348 / 11,505), w2
+// takes its K splits instead (config 3 4,820 + 129 us of combine against 6,315
+// + 39; 1,024 tokens 1,519 + 39 against 2,029 + 13; config 5 at 256 / 1,024
+// tokens 53 / 96 against 58 / 107; the reference's at 1,024 tokens level).
 int choose_sk(moe_ctx* ctx, moe::GemmUse use, int64_t pairs, int64_t E, int64_t N, int64_t K,
-              int dp_splits, int dp_slots) {
+              int dp_splits, int dp_slots, bool fp32) {
     static const int env_mode = env_int("MOE_SK", -1);
     const int env = ctx->sk_mode >= 0 ? ctx->sk_mode : env_mode;
     if (env == 0 || pairs == 0 || K % 16 != 0 || K < 32) return 0;
     const moe::GemmTile t = moe::gemm_tile(use);
     const int64_t bound_tiles = grouped_m_tiles(pairs, E, t.bm) * moe::ceil_div(N, t.bn);
     if (bound_tiles * (K / 16) > INT32_MAX) return 0;
-    int& occ = ctx->sk_blocks_per_cu[static_cast<int>(use)];
-    if (occ == 0) occ = moe::gemm_sk_blocks_per_cu(use);
-    const int slots = ctx->cus * occ;
+    const int slots = grouped_slots(ctx, use, fp32, true);
     if (env == 1) return slots;
     const double nk = double(K / 16);
     const double tiles = double(expected_m_tiles(pairs, E, t.bm) * moe::ceil_div(N, t.bn));
@@ -410,6 +439,7 @@ int choose_sk(moe_ctx* ctx, moe::GemmUse use, int64_t pairs, int64_t E, int64_t 
     const double w = tiles * S / dp_slots;
     if (w / std::ceil(w) >= 0.96) return 0;
     const bool w2 = use == moe::GemmUse::W2 || use == moe::GemmUse::W2Narrow;
+    if (!fp32 && (w2 || tiles > 0.7 * dp_slots)) return 0;
     const double left = tiles - std::floor(tiles / slots) * slots;
     if (w2 && left * nk / slots < 64) return 0;
     double G = slots;
@@ -523,26 +553,24 @@ FfnPlan choose_ffn_plan(moe_ctx* ctx, int64_t pairs, int64_t d, int64_t d_ff, in
         f.splits = 1;
         return f;
     }
-    // workgroups of the one-tile-per-workgroup kernel of `use` the GPU holds
-    auto slots_of = [&](moe::GemmUse use) {
-        int& occ = use == moe::GemmUse::W2Narrow ? ctx->w2n_blocks_per_cu
-                   : use == moe::GemmUse::W2     ? ctx->w2_blocks_per_cu
-                                                 : ctx->w13_blocks_per_cu[f.w13_tile];
-        if (occ == 0) occ = moe::gemm_blocks_per_cu(use);
-        return ctx->cus * occ;
-    };
+    f.fp32 = few_rows(pairs, E);
     const moe::GemmUse u13 = f.w13_tile == 1 ? moe::GemmUse::W13Tall : moe::GemmUse::W13;
     auto use_of = [](int tile) { return tile == 1 ? moe::GemmUse::W2Narrow : moe::GemmUse::W2; };
-    W2SplitPlan w2 = choose_w2_split_plan(ctx, pairs, d, d_ff, E, f.tile);
-    f.w13_sk = choose_sk(ctx, u13, pairs, E, d_ff, d, 1, slots_of(u13));
+    auto w2_sk = [&](int tile, int splits) {
+        return choose_sk(ctx, use_of(tile), pairs, E, d, d_ff, splits,
+                         grouped_slots(ctx, use_of(tile), f.fp32, false), f.fp32);
+    };
+    W2SplitPlan w2 = choose_w2_split_plan(ctx, pairs, d, d_ff, E, f.tile, f.fp32);
+    f.w13_sk = choose_sk(ctx, u13, pairs, E, d_ff, d, 1, grouped_slots(ctx, u13, f.fp32, false),
+                         f.fp32);
     // w2: stream-K against its best split plan
-    f.w2_sk = choose_sk(ctx, use_of(f.tile), pairs, E, d, d_ff, w2.splits, slots_of(use_of(f.tile)));
+    f.w2_sk = w2_sk(f.tile, w2.splits);
     if (!tile_pinned && f.tile == 0 && f.w2_sk == 0) {
-        const W2SplitPlan narrow = choose_w2_split_plan(ctx, pairs, d, d_ff, E, 1);
+        const W2SplitPlan narrow = choose_w2_split_plan(ctx, pairs, d, d_ff, E, 1, f.fp32);
         if (narrow.us < w2.us) {
             f.tile = 1;
             w2 = narrow;
-            f.w2_sk = choose_sk(ctx, use_of(1), pairs, E, d, d_ff, w2.splits, slots_of(use_of(1)));
+            f.w2_sk = w2_sk(1, w2.splits);
         }
     }
     f.splits = f.w2_sk > 0 ? 1 : w2.splits;
@@ -557,7 +585,7 @@ FfnPlan choose_ffn_plan(moe_ctx* ctx, int64_t pairs, int64_t d, int64_t d_ff, in
 }
 
 W2SplitPlan choose_w2_split_plan(moe_ctx* ctx, int64_t pairs, int64_t d, int64_t d_ff, int64_t E,
-                                 int w2_tile) {
+                                 int w2_tile, bool fp32) {
     static const int env = [] {
         const char* v = std::getenv("MOE_W2_SPLITS");
         return v != nullptr ? std::atoi(v) : 0;
@@ -565,23 +593,28 @@ W2SplitPlan choose_w2_split_plan(moe_ctx* ctx, int64_t pairs, int64_t d, int64_t
     auto allowed = [&](int S) { return S == 1 || (d_ff > 0 && d_ff % (16 * S) == 0); };
     const bool pinned = env == 1 || env == 2 || env == 4;
     const moe::GemmUse use = w2_tile == 1 ? moe::GemmUse::W2Narrow : moe::GemmUse::W2;
-    int& occ = w2_tile == 1 ? ctx->w2n_blocks_per_cu : ctx->w2_blocks_per_cu;
-    if (occ == 0) occ = moe::gemm_blocks_per_cu(use);
     const moe::GemmTile tile = moe::gemm_tile(use);
     // the kernel deals only real tiles: sum over experts of ceil(n_e / BM),
     // expected ceil(pairs / BM) + E / 2 (each expert's last tile half full)
     const double tiles = double(expected_m_tiles(pairs, E, tile.bm) * moe::ceil_div(d, tile.bn));
-    const double slots = double(int64_t(ctx->cus) * occ);
+    const double slots = double(grouped_slots(ctx, use, fp32, false));
     // Time of S splits: ceil(tiles * S / slots) rounds of K / S steps, plus
     // the S - 1 extra partial row buffers w2 writes and the combine reads.
     // A round of n K steps: 3.9 n + 9 us on the wide tile (64 MFMAs per wave
     // and step, two workgroups per CU), 3.2 n us on the 128 x 128 one (32,
     // three per CU): fitted to rounds measured on MI355X at n = 28 (the
-    // reference's d_ff 448), 88 (config 4) and 896 (config 3).
+    // reference's d_ff 448), 88 (config 4) and 896 (config 3).  On the bf16
+    // pieces 2.3 n + 7 and 2 n + 3 (rounds of 72 us at n = 28, 210 at 88; 58
+    // and 178), and a last round of at most one workgroup per CU takes 0.65 of
+    // a full one.
     const double nk = double(std::max<int64_t>(d_ff / 16, 1));
-    auto round_us = [&](double n) { return w2_tile == 1 ? 3.2 * n : 3.9 * n + 9.0; };
+    auto round_us = [&](double n) {
+        if (!fp32) return w2_tile == 1 ? 2.0 * n + 3.0 : 2.3 * n + 7.0;
+        return w2_tile == 1 ? 3.2 * n : 3.9 * n + 9.0;
+    };
     auto time_of = [&](int S) {
-        const double rounds = std::ceil(tiles * S / slots);
+        double rounds = std::ceil(tiles * S / slots);
+        if (!fp32 && tiles * S - (rounds - 1) * slots <= ctx->cus) rounds -= 0.35;
         return rounds * round_us(nk / S) + (S - 1) * double(pairs) * d * 8.0 / 6e6;
     };
     if (pinned) {
@@ -613,6 +646,7 @@ void expert_ffn(moe_ctx* ctx, const float* x, const int32_t* perm,
             moe::gemm_tile(f.w13_tile == 1 ? moe::GemmUse::W13Tall : moe::GemmUse::W13);
         moe::GemmArgs a{};
         a.tile = f.w13_tile;
+        a.fp32 = f.fp32;
         a.A = x;
         a.lda = d;
         a.gather = perm;
@@ -655,6 +689,7 @@ void expert_ffn(moe_ctx* ctx, const float* x, const int32_t* perm,
         moe::gemm_tile(f.tile == 1 ? moe::GemmUse::W2Narrow : moe::GemmUse::W2);
     moe::GemmArgs b{};
     b.tile = f.tile;
+    b.fp32 = f.fp32;
     b.A = d_ff > 0 ? h : out_rows;
     b.lda = d_ff;
     b.B0 = d_ff > 0 ? w2 : out_rows;
@@ -1531,9 +1566,18 @@ int moe_layer_forward_noalloc(moe_ctx* ctx, const moe_layer_desc* desc,
         if (desc->T == 0) return;
         moe::require(ctx->scratch != nullptr, "no-alloc scratch not bound to this context");
         DeviceScope dev(ctx->device);
-        const FfnPlan plan =
-            choose_ffn_plan(ctx, desc->T * desc->k, desc->d, desc->d_ff, desc->E);
-        const size_t need = carve_layer(nullptr, *desc, plan).bytes;
+        FfnPlan plan = choose_ffn_plan(ctx, desc->T * desc->k, desc->d, desc->d_ff, desc->E);
+        size_t need = carve_layer(nullptr, *desc, plan).bytes;
+        if (need > kNoAllocScratchBytes) {
+            // every tile whole: no partial tiles, no split partials
+            if (!plan.skinny13) plan.w13_sk = 0;
+            if (!plan.skinny2) {
+                plan.w2_sk = 0;
+                plan.splits = 1;
+            }
+            if (!plan.skinny13) plan.sk_floats = 0;
+            need = carve_layer(nullptr, *desc, plan).bytes;
+        }
         if (need > kNoAllocScratchBytes)
             throw moe::InvalidArg("moe_layer_forward_noalloc: this layer needs " +
                                   std::to_string(need) + " bytes of scratch, more than the " +

@@ -57,10 +57,11 @@ struct GemmTile {
     int bm, bn;
 };
 GemmTile gemm_tile(GemmUse use);
-// Workgroups of the grouped kernel of `use` one CU holds at once.
-int gemm_blocks_per_cu(GemmUse use);
+// Workgroups of the grouped kernel of `use` one CU holds at once (fp32: of
+// its fp32 MFMA form, GemmArgs::fp32).
+int gemm_blocks_per_cu(GemmUse use, bool fp32);
 // ... of its stream-K kernel (GemmArgs::sk_grid > 0).
-int gemm_sk_blocks_per_cu(GemmUse use);
+int gemm_sk_blocks_per_cu(GemmUse use, bool fp32);
 // Floats of GemmArgs::sk_part a stream-K launch of `use` on `grid`
 // workgroups needs.
 int64_t gemm_sk_part_floats(GemmUse use, int grid);
@@ -136,6 +137,9 @@ struct GemmArgs {
     // NB * BM * BN floats for the tiles their range boundaries cut.
     int32_t sk_grid;
     float* sk_part;
+    // Grouped tiles on fp32 MFMA instead of the bf16 pieces (split.hpp): the
+    // launches whose experts hold few rows, bound by reading the weights.
+    int32_t fp32;
     // Dense, one batch, no K split: a residual [M, N] with C's leading dim,
     // added after the bias, C = (A B + bias) + resid (it may be C itself);
     // nullptr for none.
@@ -253,10 +257,10 @@ void launch_combine(const float* out_rows, const int32_t* idx, const float* w,
 struct moe_ctx {
     int device = 0;
     int cus = 0;               // compute units of the device
-    int w2_blocks_per_cu = 0;  // occupancy of the grouped w2 kernel (lazily queried)
-    int w2n_blocks_per_cu = 0;  // ... of its 128x128-tile variant
-    int w13_blocks_per_cu[2] = {};  // ... of the w1/w3 kernel, per tile (GemmArgs::tile)
-    int sk_blocks_per_cu[5] = {};   // ... of the stream-K kernels, per GemmUse
+    // occupancy of the grouped kernels and of their stream-K forms, per
+    // GemmArgs::fp32 and GemmUse (lazily queried)
+    int grouped_blocks_per_cu[2][5] = {};
+    int sk_blocks_per_cu[2][5] = {};
     int sk_mode = -1;  // moe_ctx_set_stream_k: -1 planner (or MOE_SK), 0 off, 1 on
     int dense_blocks_per_cu[2][moe::kDenseTiles] = {};  // [nn][tile], lazily queried
     void* ws = nullptr;

@@ -1,4 +1,6 @@
-// fp32 GEMM engine for gfx950 on the matrix cores (v_mfma_f32_32x32x2_f32).
+// fp32 GEMM engine for gfx950 on the matrix cores: v_mfma_f32_32x32x2_f32,
+// and, for the expert tiles, v_mfma_f32_32x32x16_bf16 over three exact bf16
+// pieces of every fp32 value (split.hpp).
 //
 // One kernel template serves every contraction of the MoE path:
 //   dense NT  C = A B^T (+bias)       tensor_ops::matmul_transposed / Linear
@@ -28,6 +30,7 @@
 // and w1/w3 need no interleaved copy (the reference interleaves rows at
 // load, src/model.cu:1340-1365).
 #include "common.hpp"
+#include "split.hpp"
 
 #include <cstdlib>
 #include <type_traits>
@@ -1346,6 +1349,311 @@ __device__ __forceinline__ void direct_tile(const GemmArgs& p, int mt, int nt, i
     store_tile<C, NB, EPI>(p, Cb, split, row0, rows, n0, acc, tid);
 }
 
+// ---------------------------------------------------------------------------
+// The same tile on the bf16 matrix cores (split.hpp): fp32 rows are loaded
+// into registers, split into three bf16 planes on their way to LDS, and each
+// 32x32x16 block is six v_mfma_f32_32x32x16_bf16.
+//
+// LDS holds, per operand and stage, 3 planes x 2 halves of the 16-wide K
+// step: half h of a row is 8 bf16 (k = 8h .. 8h+7, one lane's operand), rows
+// 16 bytes apart, so a fragment read is 64 consecutive 16-byte slots; the
+// halves lie 64 bytes past a multiple of 256 apart, so the four lanes that
+// split one row's K step store to different banks.  Two stages: step kt
+// reads stage kt % 2, splits the rows of step kt + 1 (loaded during step
+// kt - 1) into the other one and starts the loads of step kt + 2; one barrier
+// per step.  The split runs once per workgroup, not once per wave that reads
+// a row: 168 vector instructions per wave and step, which issue under its 48
+// MFMAs.
+//
+// Bound: power.  The bare MFMA loop holds about 1,750 TFLOP/s of bf16 on this
+// card at 1.7 GHz; in these tiles the matrix pipe is busy 64-74 % of the cycles
+// at 1.5 GHz.  Measured on MI355X, ms per launch and fp32 TFLOP/s, on
+// v_mfma_f32_32x32x2_f32 -> here: config 3 w1/w3 13.7 (140) -> 10.3 (187), w2
+// 6.9 (139) -> 4.9 (197); config 4 w1/w3 10.9 (138) -> 7.3 (208), w2 5.5 (138)
+// -> 3.6 (209); the reference's layer w1/w3 1.75 (131) -> 1.31 (175), w2 0.91
+// (126) -> 0.57 (201).  256 x 256 tiles of 8 waves, which load and split a
+// third less per product, were no faster (config 3 12.2 and 5.2, config 4 7.8
+// and 3.7): one workgroup per CU stands still at its barriers.
+template <int ROWS>
+struct SplitPlanes {
+    static constexpr int HALF = ROWS * 16 + 64;  // bytes of one half plane
+    static constexpr int BYTES = 6 * HALF;
+    static __device__ __forceinline__ int at(int piece, int half, int row) {
+        return (piece * 2 + half) * HALF + row * 16;
+    }
+};
+
+// One 32x32 block over K columns [0, K) of the fp32 rows at `a` and `b` (this
+// lane's row lane % 32 of the block's A and B rows) on fp32 MFMA: blocks
+// whose split is not exact.
+__device__ __attribute__((noinline)) f32x16 fp32_block(const float* a, const float* b, int64_t K) {
+    const int lh = (threadIdx.x & 63) >> 5;
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    for (int64_t k = 8 * lh; k < K; k += 16) {
+        f32x4 x[2], y[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            x[q] = *reinterpret_cast<const f32x4*>(a + k + 4 * q);
+            y[q] = *reinterpret_cast<const f32x4*>(b + k + 4 * q);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[q][s], y[q][s], acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+template <class C, bool GROUPED, int NB, int EPI, bool LOOPED = false>
+__device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, int split,
+                                           int64_t seg_lo, int64_t seg_hi, float* part) {
+    constexpr int BM = C::BM, BN = C::BN, FM = C::FM, FN = C::FN, T = C::THREADS;
+    constexpr int CA = BM * 4 / T, CB = BN * 4 / T;  // 16-byte chunks per thread and step
+    static_assert(CA * T == BM * 4 && CB * T == BN * 4 && C::KW == 1, "chunk split");
+    using PA = SplitPlanes<BM>;
+    using PB = SplitPlanes<BN>;
+    constexpr int STAGE = PA::BYTES + NB * PB::BYTES;
+    __shared__ __align__(16) unsigned char S0[STAGE], S1[STAGE];
+
+    int tid = threadIdx.x;
+    if constexpr (LOOPED) asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, wave = tid >> 6;
+
+    int64_t row0;
+    int rows;
+    const float* B[NB];
+    if (GROUPED) {
+        int e;
+        if (!grouped_tile_rows<BM>(p, mt, e, row0, rows)) return;
+        B[0] = p.B0 + e * p.b_expert_stride;
+        if (NB == 2) B[NB - 1] = p.B1 + e * p.b_expert_stride;
+    } else {
+        row0 = static_cast<int64_t>(mt) * BM;
+        rows = static_cast<int>(p.M - row0 < BM ? p.M - row0 : BM);
+        B[0] = p.B0;
+        if (NB == 2) B[NB - 1] = p.B1;
+    }
+    const int64_t n0 = static_cast<int64_t>(nt) * BN;
+    const int64_t N = p.N;
+    int64_t kbeg = split * p.k_split_len;
+    int64_t K = p.K - kbeg < p.k_split_len ? p.K : kbeg + p.k_split_len;
+    if (seg_lo >= 0) {
+        K = kbeg + seg_hi * 16;
+        kbeg += seg_lo * 16;
+    }
+    const int nk = __builtin_amdgcn_readfirstlane(static_cast<int>((K - kbeg) / 16));
+
+    // A row of this tile: past the edge a valid row, masked at the store
+    auto a_row = [&](int r) -> const float* {
+        r = r < rows ? r : rows - 1;
+        int64_t src = row0 + r;
+        if (GROUPED && p.gather != nullptr) {
+            int64_t tok = p.gather[row0 + r];
+            src = tok < 0 ? 0 : (tok >= p.gather_rows ? p.gather_rows - 1 : tok);
+        }
+        return p.A + src * p.lda;
+    };
+    auto b_row = [&](int nb, int r) -> const float* {
+        const int64_t n = n0 + r < N ? n0 + r : N - 1;
+        return B[nb] + n * p.ldb;
+    };
+    // Chunk c = tid + T*i of an operand's K step: row c / 4, columns
+    // 4 (c % 4) .. + 3; byte offsets from wave-uniform bases (the host takes
+    // this path only when they stay below 2^31).
+    const float* abase = (GROUPED && p.gather != nullptr) ? p.A : p.A + row0 * p.lda;
+    uint32_t aoff[CA], boff[CB];
+#pragma unroll
+    for (int i = 0; i < CA; ++i) {
+        const int c = tid + T * i;
+        aoff[i] = static_cast<uint32_t>((a_row(c >> 2) - abase) * 4) + (c & 3) * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < CB; ++i) {
+        const int c = tid + T * i;
+        const int64_t r = n0 + (c >> 2) < N ? c >> 2 : N - 1 - n0;
+        boff[i] = static_cast<uint32_t>(r * p.ldb * 4) + (c & 3) * 16;
+    }
+    const float* bbase[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) bbase[nb] = B[nb] + n0 * p.ldb;
+
+    constexpr int CH = CA + NB * CB;
+    u32x4 st[CH];
+    auto load_chunk = [&](int i, uint32_t k_bytes) {
+        if (i < CA)
+            st[i] = __builtin_amdgcn_raw_buffer_load_b128(raw_rsrc(abase), aoff[i], k_bytes, 0);
+        else
+            st[i] = __builtin_amdgcn_raw_buffer_load_b128(raw_rsrc(bbase[(i - CA) / CB]),
+                                                          boff[(i - CA) % CB], k_bytes, 0);
+    };
+    float least = 1.0f;  // smallest magnitude this thread has split
+    auto split_chunk = [&](int i, unsigned char* stage) {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(st[i][j]);
+        least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(v[0])), __builtin_fabsf(v[1]));
+        least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(v[2])), __builtin_fabsf(v[3]));
+        uint32_t lo[3], hi[3];
+        split_pair(v[0], v[1], lo);
+        split_pair(v[2], v[3], hi);
+        const int c = tid + T * (i < CA ? i : (i - CA) % CB);
+        const int r = c >> 2, half = (c >> 1) & 1, at8 = (c & 1) * 8;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const int off = i < CA ? PA::at(q, half, r)
+                                   : PA::BYTES + (i - CA) / CB * PB::BYTES + PB::at(q, half, r);
+            *reinterpret_cast<u32x2*>(stage + off + at8) = u32x2{lo[q], hi[q]};
+        }
+    };
+    auto k_bytes = [&](int kt) {
+        kt = kt < nk ? kt : nk - 1;  // the last steps load again what no step reads
+        return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
+            static_cast<int>(static_cast<uint32_t>((kbeg + int64_t(kt) * 16) * 4))));
+    };
+
+    const int wm = wave % C::WM, wn = wave / C::WM;
+    const int lr = lane & 31, lh = lane >> 5;
+    const int arow0 = wm * (BM / C::WM), bcol0 = wn * (BN / C::WN);
+    const int live_rows = n0 + bcol0 < N ? rows - arow0 : 0;
+    const int live = live_rows <= 0 ? 0 : (live_rows >= FM * 32 ? FM : (live_rows + 31) / 32);
+
+    f32x16 acc[NB][FM][FN];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int bi = 0; bi < FM; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < FN; ++bj)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[nb][bi][bj][r] = 0.0f;
+
+    auto frag = [&](const unsigned char* stage, int off) {
+        return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(stage + off));
+    };
+    // One K step from `cur`, splitting step kt + 1 into `next`
+    auto step = [&](auto nblk, const unsigned char* cur, unsigned char* next, int kt) {
+        constexpr int NBLK = decltype(nblk)::value;
+        constexpr int QB = NB * FN;  // B blocks of the wave
+        bf16x8 a[FM][3], b[2][3];
+        auto read_b = [&](int q) {
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+                b[q & 1][s] = frag(cur, PA::BYTES + (q / FN) * PB::BYTES +
+                                            PB::at(s, lh, bcol0 + (q % FN) * 32 + lr));
+        };
+        if constexpr (NBLK > 0) {
+#pragma unroll
+            for (int s = 0; s < 3; ++s)
+#pragma unroll
+                for (int bi = 0; bi < NBLK; ++bi)
+                    a[bi][s] = frag(cur, PA::at(s, lh, arow0 + bi * 32 + lr));
+            read_b(0);
+        }
+        const uint32_t kb = k_bytes(kt + 2);
+        static_for_int(std::make_integer_sequence<int, QB>{}, [&](auto qi) {
+            constexpr int Q = decltype(qi)::value;
+            if constexpr (NBLK > 0) {
+                if constexpr (Q + 1 < QB) read_b(Q + 1);
+#pragma unroll
+                for (int t = 0; t < kSplitTerms; ++t)
+#pragma unroll
+                    for (int bi = 0; bi < NBLK; ++bi)
+                        acc[Q / FN][bi][Q % FN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            a[bi][kSplitA[t]], b[Q & 1][kSplitB[t]], acc[Q / FN][bi][Q % FN], 0, 0,
+                            0);
+            }
+            // this block's share of the next step's chunks
+            constexpr int C0 = CH * Q / QB, C1 = CH * (Q + 1) / QB;
+#pragma unroll
+            for (int i = C0; i < C1; ++i) {
+                split_chunk(i, next);
+                load_chunk(i, kb);
+            }
+        });
+        ring_barrier();
+    };
+    auto k_loop = [&](auto nblk) {
+        if (nk > 0) {
+            uint32_t kb = k_bytes(0);
+#pragma unroll
+            for (int i = 0; i < CH; ++i) load_chunk(i, kb);
+            kb = k_bytes(1);
+#pragma unroll
+            for (int i = 0; i < CH; ++i) {
+                split_chunk(i, S0);
+                load_chunk(i, kb);
+            }
+            ring_barrier();
+        }
+        for (int kt = 0; kt < nk; kt += 2) {
+            step(nblk, S0, S1, kt);
+            if (kt + 1 >= nk) break;
+            step(nblk, S1, S0, kt + 1);
+        }
+    };
+    if (live > 1 || (FM == 1 && live == 1)) k_loop(std::integral_constant<int, FM>{});
+    else if (live == 1) k_loop(std::integral_constant<int, 1>{});
+    else k_loop(std::integral_constant<int, 0>{});
+
+    // Tiles that saw a magnitude below kSplitTiny look whether it was only
+    // zeros (which split exactly); a non-zero one takes the fp32 path.
+    int tiny = 0;
+    if (__syncthreads_or(least < kSplitTiny ? 1 : 0)) {
+        for (int kt = 0; kt < nk; ++kt) {
+            const uint32_t kb = k_bytes(kt);
+#pragma unroll
+            for (int i = 0; i < CH; ++i) load_chunk(i, kb);
+#pragma unroll
+            for (int i = 0; i < CH; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float v = __builtin_fabsf(__uint_as_float(st[i][j]));
+                    tiny |= v > 0.0f && v < kSplitTiny ? 1 : 0;
+                }
+        }
+        tiny = __syncthreads_or(tiny);
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int bi = 0; bi < FM; ++bi)
+#pragma unroll
+            for (int bj = 0; bj < FN; ++bj) {
+                float z = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) z = __builtin_fmaf(acc[nb][bi][bj][r], 0.0f, z);
+                if (bi < live && (tiny || __any(!(z == 0.0f))))
+                    acc[nb][bi][bj] = fp32_block(a_row(arow0 + bi * 32 + lr) + kbeg,
+                                                 b_row(nb, bcol0 + bj * 32 + lr) + kbeg, K - kbeg);
+            }
+    if (part != nullptr) {
+        f32x4* dst = reinterpret_cast<f32x4*>(part);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int bi = 0; bi < FM; ++bi)
+#pragma unroll
+                for (int bj = 0; bj < FN; ++bj)
+#pragma unroll
+                    for (int r4 = 0; r4 < 4; ++r4)
+                        dst[sk_part_index<C, NB>(nb, bi, bj, r4, tid)] =
+                            f32x4{acc[nb][bi][bj][4 * r4], acc[nb][bi][bj][4 * r4 + 1],
+                                  acc[nb][bi][bj][4 * r4 + 2], acc[nb][bi][bj][4 * r4 + 3]};
+        return;
+    }
+    store_tile<C, NB, EPI>(p, p.C, split, row0, rows, n0, acc, tid);
+}
+
+template <class C, bool GROUPED, int NB, int EPI>
+__global__ __launch_bounds__(C::THREADS, 2) void gemm_split_kernel(const GemmArgs p) {
+    int mt, nt, split;
+    if (!launch_tile<C::BM, GROUPED>(p, mt, nt, split)) return;  // surplus workgroup
+    split_tile<C, GROUPED, NB, EPI>(p, mt, nt, split, -1, -1, nullptr);
+}
+
 template <class C, int SCHED, bool NN, bool GROUPED, int NB, int EPI>
 __global__ __launch_bounds__(C::THREADS, 2) void gemm_direct_kernel(const GemmArgs p) {
     int mt, nt, split;  // split: K range of this tile (split-K)
@@ -1403,7 +1711,8 @@ __device__ __forceinline__ int sk_begin(const SkSched& s, int w) {
     return s.base + w * s.q + (w < s.r ? w : s.r);
 }
 
-template <class C, int SCHED, int NB, int EPI>
+// FP32: the tiles on fp32 MFMA (direct_tile), else on the bf16 pieces.
+template <class C, int SCHED, int NB, int EPI, bool FP32>
 __global__ __launch_bounds__(C::THREADS, 2) void gemm_sk_kernel(const GemmArgs p) {
     const int G = static_cast<int>(gridDim.x);
     const SkSched s = sk_sched<C::BM, C::BK>(p, G);
@@ -1435,7 +1744,10 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_sk_kernel(const GemmArgs p
         }
         int mt, nt;
         tile_of(t, s.m_tiles, p.n_tiles, s.group, mt, nt);
-        direct_tile<C, SCHED, false, true, NB, EPI, true>(p, mt, nt, 0, ks, ke, part);
+        if constexpr (FP32)
+            direct_tile<C, SCHED, false, true, NB, EPI, true>(p, mt, nt, 0, ks, ke, part);
+        else
+            split_tile<C, true, NB, EPI, true>(p, mt, nt, 0, ks, ke, part);
     }
 }
 
@@ -1892,7 +2204,11 @@ void launch_cfg(const GemmArgs& a, bool vec, hipStream_t s) {
                                    dim3(C::THREADS), 0, s, a);
                 return;
             } else {
-                if (!(SCHED & SCHED_BUFLDS) || fits)
+                if (GROUPED && fits && !a.fp32) {
+                    if constexpr (GROUPED)
+                        hipLaunchKernelGGL((gemm_split_kernel<C, GROUPED, NB, EPI>), grid,
+                                           dim3(C::THREADS), 0, s, a);
+                } else if (!(SCHED & SCHED_BUFLDS) || fits)
                     hipLaunchKernelGGL((gemm_direct_kernel<C, SCHED, NN, GROUPED, NB, EPI>), grid,
                                        dim3(C::THREADS), 0, s, a);
                 else
@@ -1930,8 +2246,12 @@ void launch_sk(const GemmArgs& a, bool vec, hipStream_t s) {
         launch_cfg<C, SCHED, false, true, NB, EPI>(d, vec, s);
         return;
     }
-    hipLaunchKernelGGL((gemm_sk_kernel<C, SCHED, NB, EPI>), dim3(a.sk_grid), dim3(C::THREADS), 0,
-                       s, a);
+    if (a.fp32)
+        hipLaunchKernelGGL((gemm_sk_kernel<C, SCHED, NB, EPI, true>), dim3(a.sk_grid),
+                           dim3(C::THREADS), 0, s, a);
+    else
+        hipLaunchKernelGGL((gemm_sk_kernel<C, SCHED, NB, EPI, false>), dim3(a.sk_grid),
+                           dim3(C::THREADS), 0, s, a);
     if (a.sk_grid > 1)
         hipLaunchKernelGGL((gemm_sk_fixup_kernel<C, NB, EPI>),
                            dim3(a.sk_grid - 1, C::FM * C::FN), dim3(C::THREADS), 0, s, a);
@@ -2028,70 +2348,34 @@ int dense_blocks_per_cu(int tile, bool nn) {
     }
 }
 
-int gemm_blocks_per_cu(GemmUse use) {
+namespace {
+template <class C, int SCHED, int NB, int EPI>
+int grouped_occupancy(bool fp32, bool sk) {
     int n = 0;
-    hipError_t e = hipSuccess;
-    auto query = [&](auto kernel, int threads) {
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0);
+    auto query = [&](auto kernel) {
+        hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, C::THREADS, 0),
+                  "hipOccupancyMaxActiveBlocksPerMultiprocessor");
     };
-    switch (use) {
-        case GemmUse::W2Narrow:
-            query(gemm_direct_kernel<W2NarrowCfg, MOE_W2_SCHED | SCHED_DIRECT, false, true, 1,
-                                     EPI_STORE>,
-                  W2NarrowCfg::THREADS);
-            break;
-        case GemmUse::W2:
-            if constexpr ((MOE_W2_SCHED & SCHED_DIRECT) != 0 && W2Cfg::BK == 16)
-                query(gemm_direct_kernel<W2Cfg, MOE_W2_SCHED, false, true, 1, EPI_STORE>,
-                      W2Cfg::THREADS);
-            else
-                query(gemm_kernel<W2Cfg, MOE_W2_SCHED, false, true, true, 1, EPI_STORE>,
-                      W2Cfg::THREADS);
-            break;
-        case GemmUse::W13Tall:
-            query(gemm_direct_kernel<W13TallCfg, MOE_W13_SCHED, false, true, 2, EPI_SWIGLU>,
-                  W13TallCfg::THREADS);
-            break;
-        default:
-            if constexpr ((MOE_W13_SCHED & SCHED_DIRECT) != 0 && W13Cfg::BK == 16)
-                query(gemm_direct_kernel<W13Cfg, MOE_W13_SCHED, false, true, 2, EPI_SWIGLU>,
-                      W13Cfg::THREADS);
-            else
-                query(gemm_kernel<W13Cfg, MOE_W13_SCHED, false, true, true, 2, EPI_SWIGLU>,
-                      W13Cfg::THREADS);
-            break;
-    }
-    hip_check(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+    if (sk && fp32) query(gemm_sk_kernel<C, SCHED, NB, EPI, true>);
+    else if (sk) query(gemm_sk_kernel<C, SCHED, NB, EPI, false>);
+    else if (fp32) query(gemm_direct_kernel<C, SCHED, false, true, NB, EPI>);
+    else query(gemm_split_kernel<C, true, NB, EPI>);
     return n > 0 ? n : 1;
 }
+int grouped_occupancy(GemmUse use, bool fp32, bool sk) {
+    constexpr int S13 = MOE_W13_SCHED | SCHED_DIRECT, S2 = MOE_W2_SCHED | SCHED_DIRECT;
+    switch (use) {
+        case GemmUse::W2Narrow: return grouped_occupancy<W2NarrowCfg, S2, 1, EPI_STORE>(fp32, sk);
+        case GemmUse::W2: return grouped_occupancy<W2Cfg, S2, 1, EPI_STORE>(fp32, sk);
+        case GemmUse::W13Tall: return grouped_occupancy<W13TallCfg, S13, 2, EPI_SWIGLU>(fp32, sk);
+        default: return grouped_occupancy<W13Cfg, S13, 2, EPI_SWIGLU>(fp32, sk);
+    }
+}
+}  // namespace
 
-int gemm_sk_blocks_per_cu(GemmUse use) {
-    int n = 0;
-    hipError_t e = hipSuccess;
-    auto query = [&](auto kernel, int threads) {
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0);
-    };
-    switch (use) {
-        case GemmUse::W2Narrow:
-            query(gemm_sk_kernel<W2NarrowCfg, MOE_W2_SCHED | SCHED_DIRECT, 1, EPI_STORE>,
-                  W2NarrowCfg::THREADS);
-            break;
-        case GemmUse::W2:
-            query(gemm_sk_kernel<W2Cfg, MOE_W2_SCHED | SCHED_DIRECT, 1, EPI_STORE>,
-                  W2Cfg::THREADS);
-            break;
-        case GemmUse::W13Tall:
-            query(gemm_sk_kernel<W13TallCfg, MOE_W13_SCHED | SCHED_DIRECT, 2, EPI_SWIGLU>,
-                  W13TallCfg::THREADS);
-            break;
-        default:
-            query(gemm_sk_kernel<W13Cfg, MOE_W13_SCHED | SCHED_DIRECT, 2, EPI_SWIGLU>,
-                  W13Cfg::THREADS);
-            break;
-    }
-    hip_check(e, "hipOccupancyMaxActiveBlocksPerMultiprocessor");
-    return n > 0 ? n : 1;
-}
+int gemm_blocks_per_cu(GemmUse use, bool fp32) { return grouped_occupancy(use, fp32, false); }
+
+int gemm_sk_blocks_per_cu(GemmUse use, bool fp32) { return grouped_occupancy(use, fp32, true); }
 
 int64_t gemm_sk_part_floats(GemmUse use, int grid) {
     const GemmTile t = gemm_tile(use);
@@ -2126,11 +2410,13 @@ void launch_gemm(const GemmArgs& args, bool nn, bool grouped, int epi, bool vec,
     // per launch 5.57 -> 5.46 ms at 16,384 tokens, 1.61 -> 1.51 ms at 4,096, 0.59 -> 0.52 ms
     // at 1,024, 0.38 -> 0.22 ms at 256; bit-identical; its w1/w3 measured level or slower)
     if (env_group == 0 && grouped && epi == EPI_STORE && a.E >= 32) group = 0;
-    // ... and so does the w1/w3 over many experts while they average at most 32 rows (config
-    // 4, same box, ms per layer: 64 / 128 / 256 tokens 0.558 / 0.783 / 0.862 -> 0.503 / 0.672 /
-    // 0.817; at 64 rows per expert, 512 tokens, it was 15 % slower)
-    if (env_group == 0 && grouped && epi != EPI_STORE && a.E >= 32 && a.rows_limit <= 32 * int64_t(a.E))
-        group = 0;
+    // ... and w1/w3 on the bf16 pieces with 8 n-tiles or more: every m-tile of one stretch of
+    // weights runs at once, so the weights come from HBM once and the activations, which the
+    // Infinity Cache holds, are what is read again (same box, ms per launch, groups of 8 ->
+    // m-fastest: config 3 11.1 -> 10.1, its 1,024 tokens 3.33 -> 3.14, config 4 7.40 -> 7.17,
+    // its 4,096 / 1,024 / 509 tokens 2.15 / 0.774 / 0.622 -> 2.03 / 0.702 / 0.530; the
+    // reference's 7 n-tiles 1.31 -> 1.33)
+    if (env_group == 0 && grouped && epi != EPI_STORE && !a.fp32 && a.n_tiles >= 8) group = 0;
     if (group < 1 || group > a.m_tiles) group = a.m_tiles;
     a.group_m = group;
     if (a.k_splits <= 1) {
@@ -2231,22 +2517,22 @@ void launch_gemm(const GemmArgs& args, bool nn, bool grouped, int epi, bool vec,
     switch (epi) {
         case EPI_SWIGLU:
             if (a.tile == 1)
-                launch_cfg<W13TallCfg, MOE_W13_SCHED, false, true, 2, EPI_SWIGLU>(a, vec, s);
+                launch_cfg<W13TallCfg, MOE_W13_SCHED | SCHED_DIRECT, false, true, 2, EPI_SWIGLU>(a, vec, s);
             else
-                launch_cfg<W13Cfg, MOE_W13_SCHED, false, true, 2, EPI_SWIGLU>(a, vec, s);
+                launch_cfg<W13Cfg, MOE_W13_SCHED | SCHED_DIRECT, false, true, 2, EPI_SWIGLU>(a, vec, s);
             break;
         case EPI_SILU:
             if (a.tile == 1)
-                launch_cfg<W13TallCfg, MOE_W13_SCHED, false, true, 1, EPI_SILU>(a, vec, s);
+                launch_cfg<W13TallCfg, MOE_W13_SCHED | SCHED_DIRECT, false, true, 1, EPI_SILU>(a, vec, s);
             else
-                launch_cfg<W13Cfg, MOE_W13_SCHED, false, true, 1, EPI_SILU>(a, vec, s);
+                launch_cfg<W13Cfg, MOE_W13_SCHED | SCHED_DIRECT, false, true, 1, EPI_SILU>(a, vec, s);
             break;
         case EPI_STORE:
             if (a.tile == 1)
                 launch_cfg<W2NarrowCfg, MOE_W2_SCHED | SCHED_DIRECT, false, true, 1, EPI_STORE>(
                     a, vec, s);
             else
-                launch_cfg<W2Cfg, MOE_W2_SCHED, false, true, 1, EPI_STORE>(a, vec, s);
+                launch_cfg<W2Cfg, MOE_W2_SCHED | SCHED_DIRECT, false, true, 1, EPI_STORE>(a, vec, s);
             break;
         default: throw Unsupported("grouped GEMM epilogue");
     }

@@ -341,7 +341,9 @@ int moe_layer_forward(moe_ctx* ctx, const moe_layer_desc* desc,
  * Every call on one GPU shares that GPU's array, which keeps the last call's
  * contents: calls that overlap on one GPU (two streams, two threads, two
  * contexts) race and must be serialised by the caller.  Same arguments,
- * results and errors as moe_layer_forward otherwise. */
+ * results and errors as moe_layer_forward otherwise; a layer that fits only
+ * without K splits and stream-K partials runs without them, its sums then
+ * rounded in another order. */
 int moe_layer_forward_noalloc(moe_ctx* ctx, const moe_layer_desc* desc,
                               const moe_layer_weights* weights, const float* x,
                               float* y, int32_t* topk_idx_out, float* topk_w_out,

@@ -524,6 +524,98 @@ def test_expert_ffn_vs_oracle(ctx, torch, orc, request_reset_stream_k, T, d, E, 
     assert_close(host(out), ref, what="expert rows")
 
 
+# Enough rows per expert for the tiles on the bf16 pieces of fp32 values, at
+# the edges of their 32-row blocks and 128- and 256-row tiles, of their column
+# tiles, and at one to three 16-column K steps.
+@pytest.mark.parametrize("T,d,E,k,d_ff,act", [
+    (127, 16, 2, 1, 16, 0), (129, 32, 2, 2, 130, 1), (257, 48, 1, 1, 448, 0),
+    (161, 144, 3, 2, 144, 0), (520, 4096, 4, 2, 64, 0), (640, 64, 4, 2, 2048, 0),
+])
+def test_expert_ffn_bf16_pieces(ctx, torch, T, d, E, k, d_ff, act):
+    """Against 64-bit sums.  Each product of pieces leaves out at most 2^-26 of
+    itself and each of the 6 K / 16 accumulations rounds once, at most 2^-23 of
+    the partial sum however the matrix unit rounds: with random signs an error
+    of about 2^-23 sqrt(6 K / 16) of the result's spread, over both products
+    at most 8 times that here (the activation's derivative, the maximum over
+    the outputs)."""
+    rng = np.random.default_rng(T + d + d_ff)
+    x, w1, w3, w2, topk = _ffn_case(rng, T, d, E, k, d_ff, act)
+    order = np.argsort(topk.ravel(), kind="stable")
+    rperm = (order // k).astype(np.int32)
+    roff = np.concatenate([[0], np.cumsum(np.bincount(topk.ravel(), minlength=E))]).astype(np.int32)
+    ref = np.empty((T * k, d))
+    f8 = lambda a: a.astype(np.float64)
+    for e in range(E):
+        rows = slice(roff[e], roff[e + 1])
+        g = f8(x[rperm[rows]]) @ f8(w1[e]).T
+        h = g / (1 + np.exp(-g))
+        if act == 0:
+            h = h * (f8(x[rperm[rows]]) @ f8(w3[e]).T)
+        ref[rows] = h @ f8(w2[e]).T
+    h = torch.empty((T * k, d_ff), device="cuda")
+    out = torch.empty((T * k, d), device="cuda")
+    ctx.expert_ffn_grouped(dev(torch, x), dev(torch, rperm), dev(torch, roff), dev(torch, w1),
+                           None if w3 is None else dev(torch, w3), dev(torch, w2), k, h, out,
+                           act=act)
+    err = np.sqrt(np.mean((host(out) - ref) ** 2) / np.mean(ref ** 2))
+    assert err <= 8 * 2.0 ** -23 * np.sqrt(6 * max(d, d_ff, 16) / 16)
+
+
+def test_expert_ffn_bf16_pieces_special_values(ctx, torch, orc):
+    """Values that three bf16 pieces do not hold take fp32 products: infinities
+    and NaN reach the outputs that they reach in fp32, the largest floats do
+    not overflow, and values under the smallest piece keep their precision."""
+    rng = np.random.default_rng(5)
+    T, d, E, k, d_ff = 300, 64, 2, 1, 160
+    x, w1, w3, w2, _ = _ffn_case(rng, T, d, E, k, d_ff, 0)
+    topk = (np.arange(T) % E).astype(np.int32)[:, None]
+    x[3, 5] = np.inf
+    x[40, 7] = -np.inf
+    x[81, 0] = np.nan
+    x[122] = 3.4028e38 * np.sign(x[122])        # hi rounds past the largest float
+    w1[:, 17] = 1e-38 * np.sign(w1[:, 17])      # ... times tiny weights: ordinary sums
+    w3[:, 17] = 1e-38 * np.sign(w3[:, 17])
+    x[200] = 1e-37 * x[200]                     # lo under bf16's smallest denormal
+    x[201] = 0.0
+    w2[0, 9] = 3.4e38 * np.sign(w2[0, 9])       # sums near and past the largest float
+    roff, rperm, _ = orc.permute(topk, E)
+    ref = orc.expert_ffn(x, rperm, roff, w1, w3, w2, act=0)
+    h = torch.empty((T * k, d_ff), device="cuda")
+    out = torch.empty((T * k, d), device="cuda")
+    ctx.expert_ffn_grouped(dev(torch, x), dev(torch, rperm), dev(torch, roff), dev(torch, w1),
+                           dev(torch, w3), dev(torch, w2), k, h, out, act=0)
+    got = host(out)
+    assert np.array_equal(np.isfinite(got), np.isfinite(ref))
+    tiny = np.flatnonzero(rperm == 200)
+    assert np.all(got[np.flatnonzero(rperm == 201)] == 0)
+    ok = np.isfinite(ref).all(axis=1)
+    for r in np.flatnonzero(ok):                # each row to its own scale
+        scale = np.max(np.abs(ref[r]))
+        assert np.max(np.abs(got[r] - ref[r])) <= 1e-4 * scale + 1e-38, r
+    # x = 1e-37 N(0, 1) against weights of 0.02: the gate and up sums, about
+    # 2e-38, in 64 bits
+    hg = host(h)[tiny[0]]
+    assert np.all(np.isfinite(hg))
+
+
+def test_expert_ffn_bf16_pieces_tiny_rows(ctx, torch):
+    """w1/w3 columns that scale rows of 1e-36 back to ordinary sums: fp32 keeps
+    24 bits of such rows, their bf16 pieces would keep 8."""
+    rng = np.random.default_rng(6)
+    T, d, d_ff = 140, 96, 128
+    x = (1e-36 * rng.standard_normal((T, d))).astype(np.float32)
+    w1 = (1e36 * rng.standard_normal((1, d_ff, d))).astype(np.float32)
+    w2 = normal(rng, (1, d, d_ff), 0.02)
+    off = np.array([0, T], np.int32)
+    perm = np.arange(T, dtype=np.int32)
+    h = torch.empty((T, d_ff), device="cuda")
+    out = torch.empty((T, d), device="cuda")
+    ctx.expert_ffn_grouped(dev(torch, x), dev(torch, perm), dev(torch, off), dev(torch, w1), None,
+                           dev(torch, w2), 1, h, out, act=1)
+    g = x.astype(np.float64) @ w1[0].astype(np.float64).T
+    assert_close(host(h), g / (1 + np.exp(-g)), tol=1e-5, what="tiny rows")
+
+
 # Shapes the planner sends to the grouped skinny kernel (few rows per expert,
 # K a multiple of 16; the context's default tile dealing): config 1's experts
 # (32-row workgroups, SiLU), a decoder's last rows (8 tokens, 16-row
