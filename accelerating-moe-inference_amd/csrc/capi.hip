@@ -126,6 +126,7 @@ int env_int(const char* name, int fallback) {
 // MOE_DENSE_SPLITS pin the choice for tuning.
 struct DensePlan {
     int tile = 0, splits = 1;
+    bool fp32 = true;  // GemmArgs::fp32: not on the bf16 pieces
 };
 
 #ifndef MOE_DENSE_KW_MIN
@@ -137,9 +138,82 @@ struct DensePlan {
 
 constexpr int64_t kDenseSplitBytes = int64_t(512) << 20;  // cap on the partials
 
+// The tile and K splits of a dense product on the bf16 pieces (split.hpp) and
+// their modelled time.  A K step of r workgroups on a CU takes r times its
+// share of the matrix cores, or what one workgroup needs alone (its loads,
+// split, LDS and MFMAs in turn), from MI355X times of 16 shapes x 4 tiles x 4
+// splits: 2048^3 on 128 x 128 tiles, one per CU, 101 us; 4096^3 on 256 x 128,
+// two per CU, 660-790; 1024^3 on 64 x 128, one per CU, 35; 4096 x 1024 x 1024
+// there, two per CU, 59.  A round starts and ends in about what a 4-step
+// product (200 x 520 x 64) takes: 14, 9 and 24 us per tile.  A workgroup
+// alone takes the slower of the step times it was seen to take: they depend on
+// where the operands lie in memory (1419 x 2432 x 6720 on 128 x 128, 228
+// workgroups, 274 us in one process and 460 in the next).  With few m-tiles B comes from HBM and the steps wait
+// longer: 175 x 10816 x 7168 on 64 x 128, two per CU, 1.15 us per step.
+// Whole: K in whole steps of equal splits, as the fp32 tiles need it too; else
+// the splits are whole steps but for the last.  Up to 64 rows the product is
+// bound by reading B and the fp32 tiles, loading two steps ahead, are as fast
+// (64 x 14336 x 4096 76 us against 65-82); otherwise the pieces are taken where
+// their estimate is 5 % lower, the spread of the fp32 fit.
+struct PiecesPlan {
+    DensePlan plan;
+    double seconds = 1e30;
+};
+
+PiecesPlan plan_pieces(moe_ctx* ctx, int64_t M, int64_t N, int64_t K, bool whole) {
+    static const int env_tile = env_int("MOE_DENSE_TILE", -1);
+    static const int env_splits = env_int("MOE_DENSE_SPLITS", 0);
+    static constexpr double kStep[4] = {0.70e-6, 0.42e-6, 0.0, 1.35e-6};
+    static constexpr double kAlone[4] = {1.0e-6, 0.8e-6, 0.0, 1.6e-6};
+    static constexpr double kRound[4] = {9e-6, 4.5e-6, 0.0, 16e-6};
+    constexpr double kHbm = 5.0e12, kLaunch = 2e-6, kReduce = 2e-6;
+    PiecesPlan best;
+    for (int t : {0, 1, 3}) {
+        if (env_tile >= 0 && t != env_tile) continue;
+        // (its form for any K and alignment needs more registers than two
+        // workgroups per CU leave, and spills)
+        if (t == 3 && !whole) continue;
+        const moe::GemmTile g = moe::dense_tile(t);
+        const int64_t mt = moe::ceil_div(M, g.bm), nt = moe::ceil_div(N, g.bn);
+        // resident per CU: 38 KB (64 x 128), 51 KB and 76 KB of LDS stages
+        const int64_t occ = t == 1 ? 4 : (t == 0 ? 3 : 2);
+        const double cold = M <= 256 ? 1.2 : 1.0;
+        for (int S = 1; S <= moe::kMaxDenseSplits; S *= 2) {
+            if (env_splits > 0 && S != env_splits) continue;
+            const int64_t len = moe::ceil_div(moe::ceil_div(K, S), 16) * 16;
+            if (S > 1 && (len < 64 || (S - 1) * len >= K || (whole && K % (16 * S) != 0) ||
+                          int64_t(S) * M * N * 4 > kDenseSplitBytes))
+                continue;
+            if (mt * nt * S > INT32_MAX) continue;
+            const int64_t per_cu = moe::ceil_div(mt * nt * S, ctx->cus);
+            const double steps = double(moe::ceil_div(len, 16));
+            auto round_time = [&](int64_t r) {
+                if (r == 0) return 0.0;
+                return steps * cold * std::max(double(r) * kStep[t], kAlone[t]) + kRound[t];
+            };
+            const double t_cu = double(per_cu / occ) * round_time(occ) + round_time(per_cu % occ);
+            const double part_bytes = S > 1 ? 4.0 * S * double(M) * N : 0.0;
+            const double bytes = 4.0 * (double(M) * K + double(K) * N * mt + double(M) * N);
+            double est = std::max(t_cu, (bytes + 2 * part_bytes) / kHbm) + kLaunch;
+            if (S > 1) est += kReduce + (part_bytes + 4.0 * M * N) / 4e12 + part_bytes / kHbm;
+            if (est < best.seconds) {
+                best.seconds = est;
+                best.plan = {t, S, false};
+            }
+        }
+    }
+    return best;
+}
+
 DensePlan plan_dense(moe_ctx* ctx, bool nn, bool direct, int64_t M, int64_t N, int64_t K) {
     DensePlan best;
-    if (!direct || K == 0) return best;  // the register-staged kernel: 128 x 128, one pass
+    if (K == 0) return best;
+    if (!direct) {
+        // unaligned rows or a ragged K: the pieces take them, the fp32 tiles
+        // do not (only the register-staged 128 x 128 kernel does, and where
+        // the pieces' offsets pass 2 GiB, or NN has one column, still runs)
+        return moe::pieces_fit(nn, M, N, K) ? plan_pieces(ctx, M, N, K, false).plan : best;
+    }
     static const int env_tile = env_int("MOE_DENSE_TILE", -1);
     static const int env_splits = env_int("MOE_DENSE_SPLITS", 0);
     auto split_ok = [&](int S) {
@@ -240,8 +314,12 @@ DensePlan plan_dense(moe_ctx* ctx, bool nn, bool direct, int64_t M, int64_t N, i
     if (kw_ok && (best.splits > 1 || env_tile == moe::kDenseKwTile)) {
         best.tile = moe::kDenseKwTile;
         best.splits = 1;
+        return best;
     }
-    return best;
+    if (M <= 64) return best;
+    const PiecesPlan pieces = plan_pieces(ctx, M, N, K, true);
+    return pieces.seconds < 0.95 * best_t || (env_tile >= 0 && pieces.seconds < 1e30) ? pieces.plan
+                                                                                     : best;
 }
 
 // C = A B (+ bias) (+ resid): resid [M, N] (may be C itself) is added after
@@ -284,6 +362,7 @@ void sgemm(moe_ctx* ctx, bool nn, const float* A, const float* B,
     a.m_tiles = static_cast<int32_t>(mt);
     a.n_tiles = static_cast<int32_t>(ntl);
     a.tile = plan.tile;
+    a.fp32 = plan.fp32;
     // K == 0 leaves the kernel with no K step: C = bias (or 0) still gets written.
     if (K == 0) {
         a.A = C;  // any valid pointer; never read
@@ -300,7 +379,7 @@ void sgemm(moe_ctx* ctx, bool nn, const float* A, const float* B,
         a.bias = nullptr;
         a.resid = nullptr;
         a.k_splits = plan.splits;
-        a.k_split_len = K / plan.splits;
+        a.k_split_len = moe::ceil_div(moe::ceil_div(K, plan.splits), 16) * 16;
         a.c_split_stride = M * N;
     }
     ctx->launch(nn ? "sgemm_nn" : "sgemm_nt", s, [&] {
@@ -335,7 +414,7 @@ struct FfnPlan {
     bool skinny13 = false;  // w1/w3 on the grouped skinny kernel (choose_skinny)
     bool skinny2 = false;   // w2 on it
     int w13_splits = 1;     // K splits of the skinny w1/w3 (their raw sums in sk_part)
-    bool fp32 = false;      // the tiles on fp32 MFMA (GemmArgs::fp32, few_rows)
+    bool fp32 = false;      // the tiles on fp32 MFMA (GemmArgs::fp32): few_rows, ragged K
 };
 
 // Layers whose experts hold few rows, at most 4 on average, or 16 with up to
@@ -553,7 +632,7 @@ FfnPlan choose_ffn_plan(moe_ctx* ctx, int64_t pairs, int64_t d, int64_t d_ff, in
         f.splits = 1;
         return f;
     }
-    f.fp32 = few_rows(pairs, E);
+    f.fp32 = few_rows(pairs, E) || d % 16 != 0 || d_ff % 16 != 0;
     const moe::GemmUse u13 = f.w13_tile == 1 ? moe::GemmUse::W13Tall : moe::GemmUse::W13;
     auto use_of = [](int tile) { return tile == 1 ? moe::GemmUse::W2Narrow : moe::GemmUse::W2; };
     auto w2_sk = [&](int tile, int splits) {
@@ -646,7 +725,6 @@ void expert_ffn(moe_ctx* ctx, const float* x, const int32_t* perm,
             moe::gemm_tile(f.w13_tile == 1 ? moe::GemmUse::W13Tall : moe::GemmUse::W13);
         moe::GemmArgs a{};
         a.tile = f.w13_tile;
-        a.fp32 = f.fp32;
         a.A = x;
         a.lda = d;
         a.gather = perm;
@@ -675,6 +753,7 @@ void expert_ffn(moe_ctx* ctx, const float* x, const int32_t* perm,
             a.sk_part = sk_part;
         }
         const bool vec = d % 4 == 0 && aligned16(x) && aligned16(w1) && (!swiglu || aligned16(w3));
+        a.fp32 = f.fp32 || !vec;  // (the pieces' grouped tiles need aligned rows)
         if (f.skinny13 && !vec) {  // unaligned rows: one 128x128 tile per workgroup, K whole
             a.tile = 0;
             a.k_splits = 1;
@@ -689,7 +768,6 @@ void expert_ffn(moe_ctx* ctx, const float* x, const int32_t* perm,
         moe::gemm_tile(f.tile == 1 ? moe::GemmUse::W2Narrow : moe::GemmUse::W2);
     moe::GemmArgs b{};
     b.tile = f.tile;
-    b.fp32 = f.fp32;
     b.A = d_ff > 0 ? h : out_rows;
     b.lda = d_ff;
     b.B0 = d_ff > 0 ? w2 : out_rows;
@@ -717,6 +795,7 @@ void expert_ffn(moe_ctx* ctx, const float* x, const int32_t* perm,
     moe::require(int64_t(b.m_tiles) * b.n_tiles * std::max(f.splits, 1) <= INT32_MAX,
                  "w2 grid too large");
     const bool vec = d_ff % 4 == 0 && aligned16(h) && aligned16(w2);
+    b.fp32 = f.fp32 || !vec;
     if (f.skinny2 && !vec) b.tile = 0;  // unaligned rows: the wide tile, the same K splits
     ctx->launch("expert_w2", s, [&] { moe::launch_gemm(b, false, true, moe::EPI_STORE, vec, s); });
 }

@@ -78,6 +78,12 @@ constexpr int kDenseTiles = 6;
 // one of the tile shapes the planner's tile loop weighs).
 constexpr int kSkinnyTile = 4;
 constexpr int kDenseKwTile = 5;
+// Whether the dense tiles on the bf16 pieces take the product (of any K and
+// alignment): their 31-bit load offsets, and a column pair for NN.
+inline bool pieces_fit(bool nn, int64_t M, int64_t N, int64_t K) {
+    const int64_t lim = (int64_t(1) << 31) / 4;
+    return M > 0 && 257 * K < lim && (nn ? N >= 2 && (K + 16) * N + 128 < lim : 129 * K < lim);
+}
 GemmTile dense_tile(int tile);
 // Workgroups of dense tile shape `tile` (direct-load kernel) one CU holds at once.
 int dense_blocks_per_cu(int tile, bool nn);
@@ -137,8 +143,9 @@ struct GemmArgs {
     // NB * BM * BN floats for the tiles their range boundaries cut.
     int32_t sk_grid;
     float* sk_part;
-    // Grouped tiles on fp32 MFMA instead of the bf16 pieces (split.hpp): the
-    // launches whose experts hold few rows, bound by reading the weights.
+    // Tiles on fp32 MFMA instead of the bf16 pieces (split.hpp): the grouped
+    // launches whose experts hold few rows and the dense products where the
+    // fp32 tiles are as fast, bound by reading the weights or by latency.
     int32_t fp32;
     // Dense, one batch, no K split: a residual [M, N] with C's leading dim,
     // added after the bias, C = (A B + bias) + resid (it may be C itself);

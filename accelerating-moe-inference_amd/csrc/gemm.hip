@@ -1383,20 +1383,56 @@ struct SplitPlanes {
     }
 };
 
+// Tiles whose chunks deal evenly to their threads.  NN: B is [K, N], so a
+// thread takes 4 k-rows of two adjacent columns (8-byte loads, 512 bytes of a
+// row per wave) and stores each column's four k; with them side by side in
+// LDS, block pair (2b, 2b + 1) of a wave holds the even and the odd columns of
+// 64: block bj, lane column c is column 64 (bj / 2) + 2 c + bj % 2, and the
+// epilogue writes two adjacent columns per lane.
+template <class C, bool NN>
+constexpr bool split_tile_fits = C::KW == 1 && C::BM * 4 % C::THREADS == 0 &&
+                                 (NN ? C::THREADS == 2 * C::BN && C::FN % 2 == 0
+                                     : C::BN * 4 % C::THREADS == 0);
+
+// K steps a tile's loads run ahead of their split: two for tiles of up to 64
+// accumulators per lane, whose registers hold two steps.  (Their steps are
+// short: one workgroup alone on its CU spent 0.79 us per step waiting for
+// loads issued a step before, 0.35 us of it in the matrix cores.)
+template <class C, int NB>
+constexpr int split_prefetch = NB * C::FM * C::FN <= 4 ? 2 : 1;
+
 // One 32x32 block over K columns [0, K) of the fp32 rows at `a` and `b` (this
-// lane's row lane % 32 of the block's A and B rows) on fp32 MFMA: blocks
-// whose split is not exact.
-__device__ __attribute__((noinline)) f32x16 fp32_block(const float* a, const float* b, int64_t K) {
+// lane's row lane % 32 of the block's A and B rows; b's elements bstep floats
+// apart) on fp32 MFMA: blocks whose split is not exact.  ANY: any K and any
+// alignment, columns past K count 0.
+template <bool NN, bool ANY>
+__device__ __attribute__((noinline)) f32x16 fp32_block(const float* a, const float* b,
+                                                       int64_t bstep, int64_t K) {
     const int lh = (threadIdx.x & 63) >> 5;
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    for (int64_t k = 8 * lh; k < K; k += 16) {
+    for (int64_t k0 = 0; k0 < K; k0 += 16) {
+        const int64_t k = k0 + 8 * lh;
         f32x4 x[2], y[2];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
+            if constexpr (ANY) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const int64_t at = k + 4 * q + s;
+                    x[q][s] = at < K ? a[at] : 0.0f;
+                    y[q][s] = at < K ? b[at * bstep] : 0.0f;
+                }
+                continue;
+            }
             x[q] = *reinterpret_cast<const f32x4*>(a + k + 4 * q);
-            y[q] = *reinterpret_cast<const f32x4*>(b + k + 4 * q);
+            if constexpr (NN) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) y[q][s] = b[(k + 4 * q + s) * bstep];
+            } else {
+                y[q] = *reinterpret_cast<const f32x4*>(b + k + 4 * q);
+            }
         }
 #pragma unroll
         for (int q = 0; q < 2; ++q)
@@ -1407,12 +1443,17 @@ __device__ __attribute__((noinline)) f32x16 fp32_block(const float* a, const flo
     return acc;
 }
 
-template <class C, bool GROUPED, int NB, int EPI, bool LOOPED = false>
+// ANY: rows of any 4-byte alignment (the 16-byte loads need no more) and any
+// K: the columns past the last whole K step are loaded one by one, zeros past
+// K, and make one more step; NN also any N >= 2: the pair at an odd N's last
+// column loads the two columns that end there.
+template <class C, bool NN, bool GROUPED, int NB, int EPI, bool ANY, bool LOOPED = false>
 __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, int split,
                                            int64_t seg_lo, int64_t seg_hi, float* part) {
     constexpr int BM = C::BM, BN = C::BN, FM = C::FM, FN = C::FN, T = C::THREADS;
-    constexpr int CA = BM * 4 / T, CB = BN * 4 / T;  // 16-byte chunks per thread and step
-    static_assert(CA * T == BM * 4 && CB * T == BN * 4 && C::KW == 1, "chunk split");
+    // 16-byte chunks per thread and step; NN: one block of 4 k-rows x 2 columns
+    constexpr int CA = BM * 4 / T, CB = NN ? 1 : BN * 4 / T;
+    static_assert(split_tile_fits<C, NN> && (!NN || NB == 1), "chunk split");
     using PA = SplitPlanes<BM>;
     using PB = SplitPlanes<BN>;
     constexpr int STAGE = PA::BYTES + NB * PB::BYTES;
@@ -1445,6 +1486,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
         kbeg += seg_lo * 16;
     }
     const int nk = __builtin_amdgcn_readfirstlane(static_cast<int>((K - kbeg) / 16));
+    const int64_t ktail = kbeg + int64_t(nk) * 16;  // ANY: columns [ktail, K) after the whole steps
 
     // A row of this tile: past the edge a valid row, masked at the store
     auto a_row = [&](int r) -> const float* {
@@ -1456,63 +1498,120 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
         }
         return p.A + src * p.lda;
     };
-    auto b_row = [&](int nb, int r) -> const float* {
-        const int64_t n = n0 + r < N ? n0 + r : N - 1;
-        return B[nb] + n * p.ldb;
+    // the column of the tile in slot `c` of LDS, and its B row (NN: column)
+    auto col_of = [](int c) { return NN ? (c & ~63) + 2 * (c & 31) + ((c >> 5) & 1) : c; };
+    auto b_row = [&](int nb, int c) -> const float* {
+        const int64_t n = n0 + col_of(c) < N ? n0 + col_of(c) : N - 1;
+        return B[nb] + (NN ? n : n * p.ldb);
     };
     // Chunk c = tid + T*i of an operand's K step: row c / 4, columns
     // 4 (c % 4) .. + 3; byte offsets from wave-uniform bases (the host takes
     // this path only when they stay below 2^31).
     const float* abase = (GROUPED && p.gather != nullptr) ? p.A : p.A + row0 * p.lda;
-    uint32_t aoff[CA], boff[CB];
+    constexpr int CBO = NN ? 4 : CB;  // NN: a k-row's offset each
+    uint32_t aoff[CA], boff[CBO];
 #pragma unroll
     for (int i = 0; i < CA; ++i) {
         const int c = tid + T * i;
         aoff[i] = static_cast<uint32_t>((a_row(c >> 2) - abase) * 4) + (c & 3) * 16;
     }
+    const int kq = tid / (BN / 2), pair = tid % (BN / 2);  // NN: k-rows 4 kq .. + 3, columns 2 pair, + 1
+    const bool odd_end = ANY && NN && n0 + 2 * pair == N - 1;  // its first column comes second
 #pragma unroll
-    for (int i = 0; i < CB; ++i) {
-        const int c = tid + T * i;
-        const int64_t r = n0 + (c >> 2) < N ? c >> 2 : N - 1 - n0;
-        boff[i] = static_cast<uint32_t>(r * p.ldb * 4) + (c & 3) * 16;
+    for (int i = 0; i < CBO; ++i) {
+        if constexpr (NN) {
+            const int64_t n = n0 + 2 * pair < N - 1 ? n0 + 2 * pair : N - 2;
+            boff[i] = static_cast<uint32_t>(((4 * kq + i) * p.ldb + n) * 4);
+        } else {
+            const int c = tid + T * i;
+            const int64_t r = n0 + (c >> 2) < N ? c >> 2 : N - 1 - n0;
+            boff[i] = static_cast<uint32_t>(r * p.ldb * 4) + (c & 3) * 16;
+        }
     }
     const float* bbase[NB];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) bbase[nb] = B[nb] + n0 * p.ldb;
+    for (int nb = 0; nb < NB; ++nb) bbase[nb] = NN ? B[nb] : B[nb] + n0 * p.ldb;
 
     constexpr int CH = CA + NB * CB;
-    u32x4 st[CH];
-    auto load_chunk = [&](int i, uint32_t k_bytes) {
-        if (i < CA)
+    constexpr int PF = split_prefetch<C, NB>;
+    u32x4 stages[PF][CH + (NN ? 1 : 0)];
+    auto load_chunk = [&](int sg, int i, uint32_t k_bytes, uint32_t bk_bytes) {
+        auto& st = stages[sg];
+        if (i < CA) {
             st[i] = __builtin_amdgcn_raw_buffer_load_b128(raw_rsrc(abase), aoff[i], k_bytes, 0);
-        else
+        } else if constexpr (NN) {
+            // k-row j's two columns in word j of st[CA] (even) and st[CA + 1] (odd)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(raw_rsrc(bbase[0]), boff[j],
+                                                                     bk_bytes, 0);
+                st[CA][j] = odd_end ? v[1] : v[0];
+                st[CA + 1][j] = v[1];
+            }
+        } else {
             st[i] = __builtin_amdgcn_raw_buffer_load_b128(raw_rsrc(bbase[(i - CA) / CB]),
                                                           boff[(i - CA) % CB], k_bytes, 0);
+        }
+    };
+    // the chunk's columns of the step at ktail, zeros past K
+    auto load_tail = [&](int i) {
+        auto& st = stages[0];
+        if (NN && i >= CA) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int64_t k = ktail + 4 * kq + j, n = n0 + 2 * pair;
+                const float* row = B[0] + k * p.ldb;
+                st[CA][j] = __float_as_uint(k < K && n < N ? row[n] : 0.0f);
+                st[CA + (NN ? 1 : 0)][j] = __float_as_uint(k < K && n + 1 < N ? row[n + 1] : 0.0f);
+            }
+            return;
+        }
+        const int c = tid + T * (i < CA ? i : (i - CA) % CB);
+        const float* row = i < CA ? a_row(c >> 2) : b_row(i < CA ? 0 : (i - CA) / CB, c >> 2);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int64_t k = ktail + (c & 3) * 4 + j;
+            st[i][j] = __float_as_uint(k < K ? row[k] : 0.0f);
+        }
     };
     float least = 1.0f;  // smallest magnitude this thread has split
-    auto split_chunk = [&](int i, unsigned char* stage) {
+    // the pieces of four consecutive k of an operand's row, to `at` + 8 bytes per piece plane
+    auto split4 = [&](const u32x4& raw, unsigned char* at, int plane) {
         float v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(st[i][j]);
+        for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(raw[j]);
         least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(v[0])), __builtin_fabsf(v[1]));
         least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(v[2])), __builtin_fabsf(v[3]));
         uint32_t lo[3], hi[3];
         split_pair(v[0], v[1], lo);
         split_pair(v[2], v[3], hi);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            *reinterpret_cast<u32x2*>(at + q * plane) = u32x2{lo[q], hi[q]};
+    };
+    auto split_chunk = [&](int sg, int i, unsigned char* stage) {
+        auto& st = stages[sg];
+        if (NN && i >= CA) {
+            const int slot = (pair & ~31) * 2 + (pair & 31), at8 = (kq & 1) * 8;
+            split4(st[CA], stage + PA::BYTES + PB::at(0, kq >> 1, slot) + at8, 2 * PB::HALF);
+            split4(st[CA + (NN ? 1 : 0)], stage + PA::BYTES + PB::at(0, kq >> 1, slot + 32) + at8,
+                   2 * PB::HALF);
+            return;
+        }
         const int c = tid + T * (i < CA ? i : (i - CA) % CB);
         const int r = c >> 2, half = (c >> 1) & 1, at8 = (c & 1) * 8;
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            const int off = i < CA ? PA::at(q, half, r)
-                                   : PA::BYTES + (i - CA) / CB * PB::BYTES + PB::at(q, half, r);
-            *reinterpret_cast<u32x2*>(stage + off + at8) = u32x2{lo[q], hi[q]};
-        }
+        if (i < CA) split4(st[i], stage + PA::at(0, half, r) + at8, 2 * PA::HALF);
+        else
+            split4(st[i], stage + PA::BYTES + (i - CA) / CB * PB::BYTES + PB::at(0, half, r) + at8,
+                   2 * PB::HALF);
     };
-    auto k_bytes = [&](int kt) {
+    // byte offset of K step kt in a row of `step` floats per k (wave-uniform)
+    auto k_bytes = [&](int kt, int64_t step) {
         kt = kt < nk ? kt : nk - 1;  // the last steps load again what no step reads
         return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(
-            static_cast<int>(static_cast<uint32_t>((kbeg + int64_t(kt) * 16) * 4))));
+            static_cast<int>(static_cast<uint32_t>((kbeg + int64_t(kt) * 16) * step * 4))));
     };
+    const int64_t bstep = NN ? p.ldb : 1;
 
     const int wm = wave % C::WM, wn = wave / C::WM;
     const int lr = lane & 31, lh = lane >> 5;
@@ -1533,8 +1632,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
     auto frag = [&](const unsigned char* stage, int off) {
         return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(stage + off));
     };
-    // One K step from `cur`, splitting step kt + 1 into `next`
-    auto step = [&](auto nblk, const unsigned char* cur, unsigned char* next, int kt) {
+    // The products of one K step from `cur`; mid(q) runs after B block q's
+    auto burst = [&](auto nblk, const unsigned char* cur, auto&& mid) {
         constexpr int NBLK = decltype(nblk)::value;
         constexpr int QB = NB * FN;  // B blocks of the wave
         bf16x8 a[FM][3], b[2][3];
@@ -1552,7 +1651,6 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
                     a[bi][s] = frag(cur, PA::at(s, lh, arow0 + bi * 32 + lr));
             read_b(0);
         }
-        const uint32_t kb = k_bytes(kt + 2);
         static_for_int(std::make_integer_sequence<int, QB>{}, [&](auto qi) {
             constexpr int Q = decltype(qi)::value;
             if constexpr (NBLK > 0) {
@@ -1565,33 +1663,57 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
                             a[bi][kSplitA[t]], b[Q & 1][kSplitB[t]], acc[Q / FN][bi][Q % FN], 0, 0,
                             0);
             }
-            // this block's share of the next step's chunks
+            mid(qi);
+        });
+    };
+    // One K step from `cur`, splitting step kt + 1 into `next` from its
+    // registers `sg`, a share of its chunks under each B block's products
+    auto step = [&](auto nblk, const unsigned char* cur, unsigned char* next, int kt, int sg) {
+        const uint32_t kb = k_bytes(kt + 1 + PF, 1), bkb = NN ? k_bytes(kt + 1 + PF, bstep) : kb;
+        burst(nblk, cur, [&](auto qi) {
+            constexpr int Q = decltype(qi)::value, QB = NB * FN;
             constexpr int C0 = CH * Q / QB, C1 = CH * (Q + 1) / QB;
 #pragma unroll
             for (int i = C0; i < C1; ++i) {
-                split_chunk(i, next);
-                load_chunk(i, kb);
+                split_chunk(sg, i, next);
+                load_chunk(sg, i, kb, bkb);
             }
         });
         ring_barrier();
+        // (the two steps of a round scheduled as one block interleave worse:
+        // config 4's layer 11.5 -> 12.0 ms)
+        __builtin_amdgcn_sched_barrier(0);
     };
     auto k_loop = [&](auto nblk) {
         if (nk > 0) {
-            uint32_t kb = k_bytes(0);
 #pragma unroll
-            for (int i = 0; i < CH; ++i) load_chunk(i, kb);
-            kb = k_bytes(1);
+            for (int g = 0; g < PF; ++g) {
+#pragma unroll
+                for (int i = 0; i < CH; ++i) load_chunk(g, i, k_bytes(g, 1), k_bytes(g, bstep));
+                // in this order: the loop's waits count the loads issued since
+                asm volatile("" ::: "memory");
+            }
 #pragma unroll
             for (int i = 0; i < CH; ++i) {
-                split_chunk(i, S0);
-                load_chunk(i, kb);
+                split_chunk(0, i, S0);
+                load_chunk(0, i, k_bytes(PF, 1), k_bytes(PF, bstep));
             }
             ring_barrier();
         }
-        for (int kt = 0; kt < nk; kt += 2) {
-            step(nblk, S0, S1, kt);
-            if (kt + 1 >= nk) break;
-            step(nblk, S1, S0, kt + 1);
+        // two steps per round and no way out between them: an exit after the
+        // first made the compiler drain every load at the head of the loop
+        for (int kt = 0; kt + 1 < nk; kt += 2) {
+            step(nblk, S0, S1, kt, PF - 1);
+            step(nblk, S1, S0, kt + 1, 0);
+        }
+        if (nk & 1) step(nblk, S0, S1, nk - 1, PF - 1);
+        if (ANY && ktail < K) {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) load_tail(i);
+#pragma unroll
+            for (int i = 0; i < CH; ++i) split_chunk(0, i, S0);
+            ring_barrier();
+            burst(nblk, S0, [](auto) {});
         }
     };
     if (live > 1 || (FM == 1 && live == 1)) k_loop(std::integral_constant<int, FM>{});
@@ -1603,14 +1725,24 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
     int tiny = 0;
     if (__syncthreads_or(least < kSplitTiny ? 1 : 0)) {
         for (int kt = 0; kt < nk; ++kt) {
-            const uint32_t kb = k_bytes(kt);
 #pragma unroll
-            for (int i = 0; i < CH; ++i) load_chunk(i, kb);
+            for (int i = 0; i < CH; ++i) load_chunk(0, i, k_bytes(kt, 1), k_bytes(kt, bstep));
 #pragma unroll
-            for (int i = 0; i < CH; ++i)
+            for (int i = 0; i < CH + (NN ? 1 : 0); ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const float v = __builtin_fabsf(__uint_as_float(st[i][j]));
+                    const float v = __builtin_fabsf(__uint_as_float(stages[0][i][j]));
+                    tiny |= v > 0.0f && v < kSplitTiny ? 1 : 0;
+                }
+        }
+        if (ANY && ktail < K) {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) load_tail(i);
+#pragma unroll
+            for (int i = 0; i < CH + (NN ? 1 : 0); ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float v = __builtin_fabsf(__uint_as_float(stages[0][i][j]));
                     tiny |= v > 0.0f && v < kSplitTiny ? 1 : 0;
                 }
         }
@@ -1626,9 +1758,45 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
 #pragma unroll
                 for (int r = 0; r < 16; ++r) z = __builtin_fmaf(acc[nb][bi][bj][r], 0.0f, z);
                 if (bi < live && (tiny || __any(!(z == 0.0f))))
-                    acc[nb][bi][bj] = fp32_block(a_row(arow0 + bi * 32 + lr) + kbeg,
-                                                 b_row(nb, bcol0 + bj * 32 + lr) + kbeg, K - kbeg);
+                    acc[nb][bi][bj] = fp32_block<NN, ANY>(
+                        a_row(arow0 + bi * 32 + lr) + kbeg,
+                        b_row(nb, bcol0 + bj * 32 + lr) + kbeg * bstep, bstep, K - kbeg);
             }
+    if constexpr (NN) {
+        // two adjacent columns per lane and row: one 8-byte store where both
+        // lie inside N and the row start is aligned to it
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        const bool vec2 = p.ldc % 2 == 0 && p.c_split_stride % 2 == 0 &&
+                          (reinterpret_cast<uintptr_t>(p.C) & 7) == 0;
+#pragma unroll
+        for (int bj = 0; bj < FN; bj += 2) {
+            const int64_t n = n0 + col_of(bcol0 + bj * 32 + lr);
+            if (n >= N) continue;
+            const bool hb = EPI == EPI_BIAS && p.bias != nullptr;
+            const bool both = !ANY || n + 1 < N;
+            const f32x2 bv{hb ? p.bias[n] : 0.0f, hb && both ? p.bias[n + 1] : 0.0f};
+#pragma unroll
+            for (int bi = 0; bi < FM; ++bi)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int i = arow0 + bi * 32 + 8 * (r >> 2) + 4 * lh + (r & 3);
+                    if (i >= rows) continue;
+                    f32x2 v{acc[0][bi][bj][r], acc[0][bi][bj + 1][r]};
+                    if (hb) {
+                        v[0] = v[0] + bv[0];
+                        v[1] = v[1] + bv[1];
+                    }
+                    float* dst = p.C + split * p.c_split_stride + (row0 + i) * p.ldc + n;
+                    if (vec2 && both) {
+                        *reinterpret_cast<f32x2*>(dst) = v;
+                    } else {
+                        dst[0] = v[0];
+                        if (both) dst[1] = v[1];
+                    }
+                }
+        }
+        return;
+    }
     if (part != nullptr) {
         f32x4* dst = reinterpret_cast<f32x4*>(part);
 #pragma unroll
@@ -1647,11 +1815,11 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
     store_tile<C, NB, EPI>(p, p.C, split, row0, rows, n0, acc, tid);
 }
 
-template <class C, bool GROUPED, int NB, int EPI>
+template <class C, bool NN, bool GROUPED, int NB, int EPI, bool ANY>
 __global__ __launch_bounds__(C::THREADS, 2) void gemm_split_kernel(const GemmArgs p) {
     int mt, nt, split;
     if (!launch_tile<C::BM, GROUPED>(p, mt, nt, split)) return;  // surplus workgroup
-    split_tile<C, GROUPED, NB, EPI>(p, mt, nt, split, -1, -1, nullptr);
+    split_tile<C, NN, GROUPED, NB, EPI, ANY>(p, mt, nt, split, -1, -1, nullptr);
 }
 
 template <class C, int SCHED, bool NN, bool GROUPED, int NB, int EPI>
@@ -1747,7 +1915,7 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_sk_kernel(const GemmArgs p
         if constexpr (FP32)
             direct_tile<C, SCHED, false, true, NB, EPI, true>(p, mt, nt, 0, ks, ke, part);
         else
-            split_tile<C, true, NB, EPI, true>(p, mt, nt, 0, ks, ke, part);
+            split_tile<C, false, true, NB, EPI, false, true>(p, mt, nt, 0, ks, ke, part);
     }
 }
 
@@ -2190,10 +2358,30 @@ void launch_cfg(const GemmArgs& a, bool vec, hipStream_t s) {
     if constexpr ((SCHED & SCHED_DIRECT) != 0 && C::BK == 16) {
         const bool b_ok = !NN || (a.ldb % 4 == 0 && a.N % 4 == 0 &&
                                   reinterpret_cast<uintptr_t>(a.B0) % 16 == 0);
-        if (vec && b_ok && a.K % 16 == 0 && a.k_split_len % 16 == 0) {
-            const dim3 grid(static_cast<unsigned>(a.m_tiles) * static_cast<unsigned>(a.n_tiles) *
-                            static_cast<unsigned>(a.k_splits));
-            const bool fits = buf_offsets_fit(a, C::BM, C::BN, NN, GROUPED);
+        const bool whole = vec && b_ok && a.K % 16 == 0 && a.k_split_len % 16 == 0;
+        const bool fits = buf_offsets_fit(a, C::BM, C::BN, NN, GROUPED);
+        const dim3 grid(static_cast<unsigned>(a.m_tiles) * static_cast<unsigned>(a.n_tiles) *
+                        static_cast<unsigned>(a.k_splits));
+        if constexpr (split_tile_fits<C, NN>) {
+            // the bf16 pieces (NN: no residual, at least one column pair)
+            if (fits && !a.fp32 && (!NN || (a.resid == nullptr && a.N >= 2))) {
+                // any K and alignment: the dense tiles of up to 64 accumulators
+                // per lane (with 128 its guarded loads spill a hundred registers:
+                // 6610 x 3583 x 828 864 us against 356 on fp32 MFMA)
+                constexpr bool any = !GROUPED && C::BM < 256;
+                if (whole) {
+                    hipLaunchKernelGGL((gemm_split_kernel<C, NN, GROUPED, NB, EPI, false>), grid,
+                                       dim3(C::THREADS), 0, s, a);
+                    return;
+                }
+                if constexpr (any) {
+                    hipLaunchKernelGGL((gemm_split_kernel<C, NN, GROUPED, NB, EPI, true>), grid,
+                                       dim3(C::THREADS), 0, s, a);
+                    return;
+                }
+            }
+        }
+        if (whole) {
             if constexpr (C::KW > 1) {
                 // K groups: the ring path only, every group the same K steps
                 static_assert((SCHED & SCHED_BUFLDS) && (SCHED & SCHED_RING3), "K groups need the ring");
@@ -2204,11 +2392,7 @@ void launch_cfg(const GemmArgs& a, bool vec, hipStream_t s) {
                                    dim3(C::THREADS), 0, s, a);
                 return;
             } else {
-                if (GROUPED && fits && !a.fp32) {
-                    if constexpr (GROUPED)
-                        hipLaunchKernelGGL((gemm_split_kernel<C, GROUPED, NB, EPI>), grid,
-                                           dim3(C::THREADS), 0, s, a);
-                } else if (!(SCHED & SCHED_BUFLDS) || fits)
+                if (!(SCHED & SCHED_BUFLDS) || fits)
                     hipLaunchKernelGGL((gemm_direct_kernel<C, SCHED, NN, GROUPED, NB, EPI>), grid,
                                        dim3(C::THREADS), 0, s, a);
                 else
@@ -2359,7 +2543,7 @@ int grouped_occupancy(bool fp32, bool sk) {
     if (sk && fp32) query(gemm_sk_kernel<C, SCHED, NB, EPI, true>);
     else if (sk) query(gemm_sk_kernel<C, SCHED, NB, EPI, false>);
     else if (fp32) query(gemm_direct_kernel<C, SCHED, false, true, NB, EPI>);
-    else query(gemm_split_kernel<C, true, NB, EPI>);
+    else query(gemm_split_kernel<C, false, true, NB, EPI, false>);
     return n > 0 ? n : 1;
 }
 int grouped_occupancy(GemmUse use, bool fp32, bool sk) {

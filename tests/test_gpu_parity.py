@@ -616,6 +616,87 @@ def test_expert_ffn_bf16_pieces_tiny_rows(ctx, torch):
     assert_close(host(h), g / (1 + np.exp(-g)), tol=1e-5, what="tiny rows")
 
 
+# The dense tiles on the bf16 pieces where they can go wrong: rows and columns
+# past the edges of the 64, 128 and 256 wide tiles, an odd last column of a
+# row-major B, K of less than one step, of whole steps and with a tail, K splits
+# whose last one is short, and operands at any 4-byte alignment.
+@pytest.mark.parametrize("layout,M,N,K,offset", [
+    ("nn", 66, 2, 5, 0), ("nn", 130, 129, 17, 1), ("nn", 200, 131, 33, 0), ("nn", 1000, 127, 16, 3),
+    ("nn", 77, 1001, 2050, 1), ("nn", 300, 640, 48, 0), ("nn", 96, 130, 4100, 0),
+    ("nt", 65, 1, 15, 1), ("nt", 129, 130, 31, 0), ("nt", 257, 255, 100, 2),
+    ("nt", 40, 300, 3001, 1), ("nt", 513, 640, 64, 0), ("nt", 2049, 1025, 32, 0),
+])
+@pytest.mark.parametrize("bias", [False, True])
+def test_sgemm_bf16_pieces(ctx, torch, layout, M, N, K, offset, bias):
+    """Against 64-bit sums, to the error the accumulations may leave (see
+    test_expert_ffn_bf16_pieces); the residual of NT too; nothing written past
+    the output."""
+    rng = np.random.default_rng(M * 31 + N * 7 + K)
+
+    def shifted(a):
+        buf = torch.zeros(a.size + offset + 8, device="cuda")
+        buf[offset:offset + a.size] = dev(torch, a).reshape(-1)
+        return buf[offset:offset + a.size].view(*a.shape)
+
+    a = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    b = rng.uniform(-1, 1, (K, N) if layout == "nn" else (N, K)).astype(np.float32)
+    bv = rng.uniform(-1, 1, N).astype(np.float32) if bias else None
+    res = rng.uniform(-1, 1, (M, N)).astype(np.float32) if layout == "nt" and bias else None
+    out = torch.full((M * N + 64,), 7.0, device="cuda")
+    c = out[:M * N].view(M, N)
+    kw = {"bias": None if bv is None else dev(torch, bv)}
+    if res is not None:
+        kw["residual"] = dev(torch, res)
+    (ctx.sgemm_nn if layout == "nn" else ctx.sgemm_nt)(shifted(a), shifted(b), c, **kw)
+    ref = a.astype(np.float64) @ (b if layout == "nn" else b.T).astype(np.float64)
+    scale = np.sqrt(np.mean(ref ** 2))
+    if bias:
+        ref = ref + bv
+    if res is not None:
+        ref = ref + res
+    err = np.sqrt(np.mean((host(c) - ref) ** 2)) / max(scale, np.sqrt(np.mean(ref ** 2)))
+    assert err <= 4 * 2.0 ** -23 * max(1.0, np.sqrt(6 * K / 16))
+    assert bool((out[M * N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("layout,N,K", [("nt", 130, 64), ("nt", 129, 70), ("nn", 132, 64),
+                                        ("nn", 131, 37)])
+def test_sgemm_bf16_pieces_special_values(ctx, torch, orc, layout, N, K):
+    """Infinities, NaN, the largest floats and values below the smallest piece
+    give what fp32 products give."""
+    rng = np.random.default_rng(N + K)
+    M = 140
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = rng.standard_normal((N, K)).astype(np.float32)
+    a[1, 3], a[33, K - 1], a[70, 0] = np.inf, np.nan, -np.inf
+    a[100] = 3.4028e38 * np.sign(a[100])
+    a[120] *= np.float32(1e-37)
+    a[139] = 0.0
+    b[5] *= np.float32(1e-38)
+    b[7] = 1e37 * b[7]
+    c = torch.empty((M, N), device="cuda")
+    if layout == "nt":
+        ctx.sgemm_nt(dev(torch, a), dev(torch, b), c)
+    else:
+        ctx.sgemm_nn(dev(torch, a), dev(torch, np.ascontiguousarray(b.T)), c)
+    got, ref = host(c), orc.matmul_nt(a, b)
+    # rows of 3.4e38: partial sums overflow in some orders and not in others
+    rows = np.r_[0:100, 101:M]
+    assert np.array_equal(np.isfinite(got[rows]), np.isfinite(ref[rows]))
+    assert np.array_equal(np.isnan(got[rows]), np.isnan(ref[rows]))
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    bound = np.abs(np.nan_to_num(a, nan=0, posinf=0, neginf=0)).astype(np.float64) @ \
+        np.abs(b).astype(np.float64).T
+    ok = np.isfinite(ref)
+    ok[100] = False
+    # each element to the sum of its products' magnitudes, and fp32's smallest step
+    with np.errstate(invalid="ignore"):
+        diff = np.abs(got - exact)
+    assert np.all(diff[ok] <= (2.0 ** -22 * K * bound + K * 2.0 ** -149)[ok])
+    big = np.abs(a[100]).astype(np.float64) @ np.abs(b[5]).astype(np.float64)
+    assert abs(got[100, 5] - exact[100, 5]) <= 2.0 ** -22 * K * big
+
+
 # Shapes the planner sends to the grouped skinny kernel (few rows per expert,
 # K a multiple of 16; the context's default tile dealing): config 1's experts
 # (32-row workgroups, SiLU), a decoder's last rows (8 tokens, 16-row
