@@ -1,5 +1,5 @@
-// Causal attention in one pass per (sequence, head, 128-query tile): the
-// scores never leave the chip.
+// Causal attention in one pass per (sequence, head, tile of 128 or 256
+// queries): the scores never leave the chip.
 //
 // Each wave owns 32 queries.  It computes the transposed scores
 // S^T[key][query] = K Q^T on fp32 MFMA (32x32x2), so the accumulator column,
@@ -24,6 +24,7 @@
 // the fp64 exp took about half as long as the MFMAs of a key block.  For the
 // same reason the division by sqrt(hd) is folded into that multiply.
 #include "common.hpp"
+#include "split.hpp"
 
 #include <cmath>
 
@@ -33,28 +34,22 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kQTile = 128;  // queries per workgroup (4 waves x 32)
 constexpr int kKBlock = 32;  // keys per block
 
-// At least two waves per SIMD: at most 256 registers a lane, which keeps
-// head_dim 128 at two waves (it took 289 and one wave) and keeps the
-// accumulators in VGPRs, where the rescale needs no AGPR moves.
-template <int HD>
-__global__ __launch_bounds__(256, 2) void flash_attn_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    float* __restrict__ out, int64_t S, int64_t H, int64_t KVH, int64_t window, float scale) {
-    static_assert(HD % 32 == 0 && HD <= 128, "head_dim 32, 64, 96 or 128");
-    constexpr int LD = HD + 8;      // LDS row stride: the lane halves land 32 banks apart
-    constexpr int QK = HD / 2;      // MFMA steps of the score product (2 dims each)
-    constexpr int MB = HD / 32;     // 32-dim blocks of the output
-    // two K/V buffers: block j is staged into buffer j % 2 while the waves
-    // read block j - 1 from the other, so one barrier per block suffices
-    __shared__ __align__(16) float Ks[2][kKBlock * LD];
-    __shared__ __align__(16) float Vs[2][kKBlock * LD];
+// What a workgroup works on, from its place in the grid.
+struct FlashTile {
+    int64_t qw, kw;        // row widths of q and out, k and v
+    const float *q, *k, *v;  // this sequence's first row, at this head's columns
+    float* out;
+    int row0;              // first query
+    int S, W;              // sequence length, window (0: none); both fit 32 bits
+    int k_lo, k_hi;        // keys the tile's queries can see
+};
 
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches
-    const int lq = lane & 31, half = lane >> 5;
+template <int HD, int NW>
+__device__ __forceinline__ FlashTile flash_tile(const float* q, const float* k, const float* v,
+                                                float* out, int64_t S, int64_t H, int64_t KVH,
+                                                int64_t window) {
     // Causal work grows with the tile index (tile t walks 4t + 4 key blocks).
     // Workgroups half a grid apart share a CU when the grid fills two per CU
     // (the dispatcher deals ids round-robin over the XCDs and their CUs), so
@@ -64,22 +59,102 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(
     const int64_t T = gridDim.x, BH = gridDim.y;
     const int64_t L = static_cast<int64_t>(blockIdx.y) * T + blockIdx.x;
     const int64_t rank = L / BH, z = L % BH;
-    const int tile = static_cast<int>(rank < (T + 1) / 2 ? T - 1 - rank : rank - (T + 1) / 2);
+    // (8 waves: one workgroup per CU, heaviest first)
+    const int tile = static_cast<int>(NW == 8 || rank < (T + 1) / 2 ? T - 1 - rank
+                                                                    : rank - (T + 1) / 2);
+    constexpr int kQTile = 32 * NW;
     const int64_t b = z / H, h = z % H, kh = h / (H / KVH);
-    const int64_t qw = H * HD, kw = KVH * HD;
-    // key and query indices fit 32 bits (the launcher checks seq_len)
-    const int S32 = static_cast<int>(S), W = static_cast<int>(window);
-    const int row0 = tile * kQTile;
-    const int q0 = row0 + 32 * wave;                  // this wave's first query
+    FlashTile t;
+    t.qw = H * HD;
+    t.kw = KVH * HD;
+    t.q = q + b * S * t.qw + h * HD;
+    t.k = k + b * S * t.kw + kh * HD;
+    t.v = v + b * S * t.kw + kh * HD;
+    t.out = out + b * S * t.qw + h * HD;
+    t.row0 = tile * kQTile;
+    t.S = static_cast<int>(S);
+    t.W = static_cast<int>(window);
+    t.k_hi = t.row0 + kQTile < t.S ? t.row0 + kQTile : t.S;
+    t.k_lo = 0;
+    if (t.W > 0 && t.row0 - (t.W - 1) > 0) t.k_lo = ((t.row0 - (t.W - 1)) / kKBlock) * kKBlock;
+    return t;
+}
+
+// The online softmax of one key block's transposed scores s (this lane's
+// query qi, register r = key k0 + 8*(r/4) + 4*half + r%4), replaced by their
+// weights; c2 = log2(e) / sqrt(hd).  `full`: every key visible.  The running
+// maximum follows the scores only once they pass it by LAG / c2, so weights
+// reach 2^LAG (their ratios, all that counts, keep every bit) and the sums are
+// rescaled by alpha in few blocks.  Returns whether any lane's are.  (A sum
+// that only a lag overflows sends the pieces' tile to fp32 MFMA, which has none.)
+template <int LAG>
+__device__ __forceinline__ bool softmax_block(f32x16& s, bool full, int k0, int qi, int half,
+                                               int S, int W, float c2, float& m_run, float& den,
+                                               float& alpha) {
+    if (!full) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int key = k0 + 8 * (r / 4) + 4 * half + (r % 4);
+            const bool vis = key <= qi && key < S && (W <= 0 || qi - key < W);
+            s[r] = vis ? s[r] : -INFINITY;
+        }
+    }
+    float bmax = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) bmax = fmaxf(bmax, s[r]);
+    bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
+    // (from -inf, nothing visible yet, any visible score moves it; NaN never)
+    const float m_new = LAG == 0                        ? fmaxf(m_run, bmax)
+                        : (bmax - m_run) * c2 > float(LAG) ? bmax
+                                                           : m_run;
+    // rescale of the sums so far (none yet, or nothing visible: 1)
+    alpha = m_run == -INFINITY || m_new == -INFINITY
+                ? 1.0f
+                : __builtin_amdgcn_exp2f((m_run - m_new) * c2);
+    // a query with nothing visible yet has m_new = -inf: its masked
+    // scores give weight 0
+    const float mc = m_new == -INFINITY ? 0.0f : m_new * c2;
+    float psum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c2, -mc));
+        psum += s[r];
+    }
+    den = den * alpha + psum;
+    m_run = m_new;
+    return __any(alpha != 1.0f);
+}
+
+// The tile on fp32 MFMA: what the pieces below leave to it (values their
+// split does not hold).  `smem`: kFp32Lds<HD> bytes.
+template <int HD>
+constexpr int kFp32Lds = 4 * kKBlock * (HD + 8) * 4;
+
+template <int HD, int NW>
+__device__ __forceinline__ void flash_fp32(const FlashTile& ft, float c2, unsigned char* smem) {
+    static_assert(HD % 32 == 0 && HD <= 128, "head_dim 32, 64, 96 or 128");
+    constexpr int LD = HD + 8;      // LDS row stride: the lane halves land 32 banks apart
+    constexpr int QK = HD / 2;      // MFMA steps of the score product (2 dims each)
+    constexpr int MB = HD / 32;     // 32-dim blocks of the output
+    // two K/V buffers: block j is staged into buffer j % 2 while the waves
+    // read block j - 1 from the other, so one barrier per block suffices
+    auto Ks = reinterpret_cast<float(*)[kKBlock * LD]>(smem);
+    auto Vs = Ks + 2;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar branches
+    const int lq = lane & 31, half = lane >> 5;
+    const int64_t kw = ft.kw;
+    const int S32 = ft.S, W = ft.W, k_lo = ft.k_lo, k_hi = ft.k_hi;
+    const int q0 = ft.row0 + 32 * wave;               // this wave's first query
     const int qi = q0 + lq;                           // this lane's query
     const bool wave_live = q0 < S32;
-    const float* kb = k + b * S * kw + kh * HD;
-    const float* vb = v + b * S * kw + kh * HD;
+    const float *kb = ft.k, *vb = ft.v;
 
     // Q^T operand: step j, half h supplies dim h*QK + j of this lane's query
     float qr[QK];
     {
-        const float* qrow = q + (b * S + (qi < S32 ? qi : S32 - 1)) * qw + h * HD + half * QK;
+        const float* qrow = ft.q + (qi < S32 ? qi : S32 - 1) * ft.qw + half * QK;
 #pragma unroll
         for (int j = 0; j < QK; j += 4) {
             const f32x4 t = *reinterpret_cast<const f32x4*>(qrow + j);
@@ -90,19 +165,14 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(
         }
     }
 
-    // keys this tile can see: [k_lo, k_hi)
-    const int k_hi = (row0 + kQTile < S32 ? row0 + kQTile : S32);
-    int k_lo = 0;
-    if (W > 0 && row0 - (W - 1) > 0) k_lo = ((row0 - (W - 1)) / kKBlock) * kKBlock;
-
     // block staging: 32 keys x HD floats of K and of V, 16-byte chunks
     constexpr int CHUNKS = kKBlock * HD / 4;       // per matrix
-    constexpr int PER_T = (CHUNKS + 255) / 256;
+    constexpr int PER_T = (CHUNKS + 64 * NW - 1) / (64 * NW);
     f32x4 kst[PER_T], vst[PER_T];
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int i = 0; i < PER_T; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c < CHUNKS) {
                 const int r = c / (HD / 4), col = 4 * (c % (HD / 4));
                 int key = k0 + r;
@@ -115,7 +185,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(
     auto stage = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < PER_T; ++i) {
-            const int c = tid + 256 * i;
+            const int c = tid + 64 * NW * i;
             if (c < CHUNKS) {
                 const int r = c / (HD / 4), col = 4 * (c % (HD / 4));
                 *reinterpret_cast<f32x4*>(&Ks[buf][r * LD + col]) = kst[i];
@@ -129,10 +199,6 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(
     for (int m = 0; m < MB; ++m)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[m][r] = 0.0f;
-    // the running maximum is kept on the unscaled scores: s / scale is
-    // monotone in s, so exp(s/scale - m/scale) = exp2((s - m) * c) with
-    // c = log2(e) / scale, one multiply per weight instead of a division
-    const float c2 = 1.44269504088896340736f / scale;
     float m_run = -INFINITY, den = 0.0f;
     const int wq_last = q0 + 31 < S32 ? q0 + 31 : S32 - 1;  // the wave's last query
 
@@ -163,38 +229,13 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(
             // every key of the block visible to every query of the wave:
             // no mask (wave-uniform)
             const bool full = k0 + kKBlock - 1 <= q0 && (W <= 0 || wq_last - k0 < W);
-            if (!full) {
+            float alpha;
+            if (softmax_block<0>(s, full, k0, qi, half, S32, W, c2, m_run, den, alpha)) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = k0 + 8 * (r / 4) + 4 * half + (r % 4);
-                    const bool vis = key <= qi && key < S32 && (W <= 0 || qi - key < W);
-                    s[r] = vis ? s[r] : -INFINITY;
-                }
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[m][r] *= alpha;
             }
-            float bmax = s[0];
-#pragma unroll
-            for (int r = 1; r < 16; ++r) bmax = fmaxf(bmax, s[r]);
-            bmax = fmaxf(bmax, __shfl_xor(bmax, 32, 64));
-            const float m_new = fmaxf(m_run, bmax);
-            // rescale of the sums so far (none yet, or nothing visible: 1)
-            const float alpha = m_run == -INFINITY || m_new == -INFINITY
-                                    ? 1.0f
-                                    : __builtin_amdgcn_exp2f((m_run - m_new) * c2);
-            // a query with nothing visible yet has m_new = -inf: its masked
-            // scores give weight 0
-            const float mc = m_new == -INFINITY ? 0.0f : m_new * c2;
-            float psum = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], c2, -mc));
-                psum += s[r];
-            }
-            den = den * alpha + psum;
-            m_run = m_new;
-#pragma unroll
-            for (int m = 0; m < MB; ++m)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[m][r] *= alpha;
             // O^T += V^T P^T: step j takes key 8*(j/4) + 4*half + j%4
             const float* vcol = &Vs[buf][lq];
 #pragma unroll
@@ -215,7 +256,7 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(
     // 32m + 8*(r/4) + 4*half + r%4: four consecutive dims per group
     const float den_all = den + __shfl_xor(den, 32, 64);
     if (wave_live && qi < S32) {
-        float* orow = out + (b * S + qi) * qw + h * HD;
+        float* orow = ft.out + qi * ft.qw;
 #pragma unroll
         for (int m = 0; m < MB; ++m)
 #pragma unroll
@@ -228,23 +269,317 @@ __global__ __launch_bounds__(256, 2) void flash_attn_kernel(
     }
 }
 
+// The tile on the bf16 pieces (split.hpp): keys and values are split once per
+// workgroup on their way to LDS, the queries once into registers, the softmax
+// weights (lane-local, as above) in registers; S^T = K Q^T and O^T += V^T P^T
+// run on v_mfma_f32_32x32x16_bf16, six per 16 dims or keys.
+//
+// K planes: per piece, 16-dim chunk and half of it, 32 keys of 16 bytes (8
+// dims, one lane's operand).  V planes are transposed: per piece, 16-key chunk
+// c and lane half h, HD dims of 16 bytes, the 8 keys 16c + 8*(j/4) + 4h + j%4
+// that registers 8c .. 8c+7 of the scores hold in that half, so P^T again goes
+// to the MFMA as it comes.  A thread takes 4 keys of two adjacent dims (the
+// even one in the first 32 slots of 64 dims, the odd one in the next 32, so
+// neighbouring lanes store side by side): accumulator block 2b + e, row i is
+// dim 64b + 2i + e.  The next block's rows are in flight in registers while a
+// block is computed.  Four waves keep one stage of planes (26 KB at head_dim
+// 64), written between two barriers while the CU's other workgroup computes;
+// eight keep two (101 KB at head_dim 128).
+//
+// Bound: the waves' own chain, scores -> softmax -> weights -> output; at
+// head_dim 128 a wave's block is 96 MFMAs (3,072 cycles) and about 390 vector
+// instructions (1,560), and two waves share a SIMD.  Measured on MI355X, fp32
+// MFMA -> here: 2 x 2047 queries, 32 heads of 128, 689 -> 383 us (100 -> 179
+// TFLOP/s); 4 x 2048, 16 heads, window 512, 366 -> 230; 2 x 2048, 32 heads of
+// 64, 315 -> 187; 8 x 512, 16 heads of 64, 54.4 -> 48.2.  Error against 64 bits
+// 3.1e-7 -> 2.6e-7, 2.9e-7 -> 2.4e-7, 3.0e-7 -> 2.5e-7, 1.8e-7 -> 1.5e-7.  The lagging
+// maximum took the first from 516 to 505 us on four waves, eight waves to 377.
+//
+// Weights under 2^-100 lose low bits (an error of at most 2^-134 of the
+// largest value); keys, values and queries under it take the fp32 tile.
+template <int HD>
+struct FlashPlanes {
+    static constexpr int KH = kKBlock * 16 + 16;  // bytes of a K half plane
+    static constexpr int VH = HD * 16 + 64;       // ... of a V one
+    static constexpr int V0 = 3 * (HD / 16) * 2 * KH;
+    static constexpr int BYTES = V0 + 12 * VH;
+    static __device__ __forceinline__ int k_at(int piece, int ch, int half, int key) {
+        return ((piece * (HD / 16) + ch) * 2 + half) * KH + key * 16;
+    }
+    static __device__ __forceinline__ int v_at(int piece, int c, int half, int slot) {
+        return V0 + ((piece * 2 + c) * 2 + half) * VH + slot * 16;
+    }
+};
+
+// Returns whether every value of the tile was split exactly and its sums came
+// out finite; the output is written only then.
+template <int HD, int NW>
+__device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsigned char* smem) {
+    constexpr int T = 64 * NW;
+    constexpr int NBUF = NW == 8 ? 2 : 1;  // stages of planes
+    using PL = FlashPlanes<HD>;
+    constexpr int CH = HD / 16;   // 16-dim chunks
+    constexpr int MB = HD / 32;   // 32-dim blocks of the output
+    constexpr int KC = kKBlock * HD / 4 / T;  // 16-byte chunks of K per thread
+    // 4-key x 2-dim blocks of V per thread; where there are fewer of them than
+    // threads, the first VN threads (whole waves) take one each
+    constexpr int VN = kKBlock * HD / 8, VC = VN >= T ? VN / T : 1;
+    auto v_mine = [&](int c) { return VN >= T || c < VN; };
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lq = lane & 31, half = lane >> 5;
+    const int S = ft.S, W = ft.W;
+    const int q0 = ft.row0 + 32 * wave, qi = q0 + lq;
+    const bool wave_live = q0 < S;
+    const int wq_last = q0 + 31 < S ? q0 + 31 : S - 1;
+    float least = 1.0f;  // smallest magnitude this thread has split
+    auto seen = [&](float a, float b) {
+        least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(a)), __builtin_fabsf(b));
+    };
+
+    // Q^T operand of chunk ch: dims 16 ch + 8 half .. + 7 of this lane's query
+    const float* qrow = ft.q + (qi < S ? qi : S - 1) * ft.qw + 8 * half;
+    u32x4 qp[CH][3];
+#pragma unroll
+    for (int ch = 0; ch < CH; ++ch)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const f32x2 x = *reinterpret_cast<const f32x2*>(qrow + 16 * ch + 2 * p);
+            uint32_t w[3];
+            seen(x[0], x[1]);
+            split_pair(x[0], x[1], w);
+#pragma unroll
+            for (int t = 0; t < 3; ++t) qp[ch][t][p] = w[t];
+        }
+
+    f32x4 kst[KC];
+    f32x2 vst[VC][4];
+    // rows k0 .. k0 + 31 from wave-uniform bases, 32-bit lane offsets; keys past
+    // the end: the last row, masked
+    const uint32_t kw4 = static_cast<uint32_t>(ft.kw) * 4;
+    auto fetch = [&](int k0) {
+        const char* kb = reinterpret_cast<const char*>(ft.k + static_cast<int64_t>(k0) * ft.kw);
+        const char* vb = reinterpret_cast<const char*>(ft.v + static_cast<int64_t>(k0) * ft.kw);
+        const int lim = S - 1 - k0;
+        auto row = [&](int r) { return static_cast<uint32_t>(r < lim ? r : lim) * kw4; };
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+            const int c = tid + T * i;
+            kst[i] = *reinterpret_cast<const f32x4*>(kb + (row(c / (HD / 4)) + 16 * (c % (HD / 4))));
+        }
+#pragma unroll
+        for (int i = 0; i < VC; ++i) {
+            const int c = tid + T * i;
+            if (!v_mine(c)) break;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                vst[i][j] = *reinterpret_cast<const f32x2*>(
+                    vb + (row(4 * (c / (HD / 2)) + j) + 8 * (c % (HD / 2))));
+        }
+    };
+    auto store4 = [&](const f32x4& x, unsigned char* at, int plane) {
+        uint32_t a[3], b[3];
+        seen(x[0], x[1]);
+        seen(x[2], x[3]);
+        split_pair(x[0], x[1], a);
+        split_pair(x[2], x[3], b);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) *reinterpret_cast<u32x2*>(at + t * plane) = u32x2{a[t], b[t]};
+    };
+    auto stage = [&](unsigned char* to) {
+#pragma unroll
+        for (int i = 0; i < KC; ++i) {
+            const int c = tid + T * i, key = c / (HD / 4), col = 4 * (c % (HD / 4));
+            store4(kst[i], to + PL::k_at(0, col / 16, (col / 8) & 1, key) + (col & 4) * 2, CH * 2 * PL::KH);
+        }
+#pragma unroll
+        for (int i = 0; i < VC; ++i) {
+            const int c = tid + T * i, kg = c / (HD / 2), dp = c % (HD / 2);
+            if (!v_mine(c)) break;
+            const int slot = (dp & ~31) * 2 + (dp & 31);
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                store4(f32x4{vst[i][0][e], vst[i][1][e], vst[i][2][e], vst[i][3][e]},
+                       to + PL::v_at(0, kg / 4, kg & 1, slot + 32 * e) + (kg & 2) * 4, 4 * PL::VH);
+        }
+    };
+    const unsigned char* cur = smem;
+    auto frag = [&](int at) {
+        return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(cur + at));
+    };
+
+    f32x16 acc[MB];
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[m][r] = 0.0f;
+    float m_run = -INFINITY, den = 0.0f;
+
+    fetch(ft.k_lo);
+    for (int k0 = ft.k_lo; k0 < ft.k_hi; k0 += kKBlock) {
+        // one stage: the previous block's planes have been read; two: the ones
+        // written now were read before the previous block's barrier
+        if (NBUF == 1) __syncthreads();
+        unsigned char* to = smem + (NBUF == 2 && ((k0 / kKBlock) & 1) ? PL::BYTES : 0);
+        stage(to);
+        __syncthreads();
+        cur = to;
+        if (k0 + kKBlock < ft.k_hi) fetch(k0 + kKBlock);
+        bool active = wave_live && k0 <= wq_last;
+        if (W > 0 && k0 + kKBlock - 1 < q0 - (W - 1)) active = false;
+        if (!active) continue;
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch) {
+            bf16x8 kp[3];
+#pragma unroll
+            for (int t = 0; t < 3; ++t) kp[t] = frag(PL::k_at(t, ch, half, lq));
+#pragma unroll
+            for (int t = 0; t < kSplitTerms; ++t)
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    kp[kSplitA[t]], __builtin_bit_cast(bf16x8, qp[ch][kSplitB[t]]), s, 0, 0, 0);
+        }
+        const bool full = k0 + kKBlock - 1 <= q0 && (W <= 0 || wq_last - k0 < W);
+        float alpha;
+        if (softmax_block<8>(s, full, k0, qi, half, S, W, c2, m_run, den, alpha)) {
+#pragma unroll
+            for (int m = 0; m < MB; ++m)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[m][r] *= alpha;
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            u32x4 pp[3];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                uint32_t w[3];
+                split_pair(s[8 * c + 2 * p], s[8 * c + 2 * p + 1], w);
+#pragma unroll
+                for (int t = 0; t < 3; ++t) pp[t][p] = w[t];
+            }
+#pragma unroll
+            for (int m = 0; m < MB; ++m) {
+                bf16x8 vp[3];
+#pragma unroll
+                for (int t = 0; t < 3; ++t) vp[t] = frag(PL::v_at(t, c, half, 32 * m + lq));
+#pragma unroll
+                for (int t = 0; t < kSplitTerms; ++t)
+                    acc[m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        vp[kSplitA[t]], __builtin_bit_cast(bf16x8, pp[kSplitB[t]]), acc[m], 0, 0, 0);
+            }
+        }
+    }
+
+    // Values the pieces do not hold: non-finite sums, and non-zero magnitudes
+    // below kSplitTiny (zeros split exactly, so a tile that saw less looks again)
+    const float den_all = den + __shfl_xor(den, 32, 64);
+    int bad = 0;
+    if (wave_live && qi < S) {
+        float z = den_all * 0.0f;
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z = fmaf(acc[m][r], 0.0f, z);
+        bad = !(z == 0.0f);
+    }
+    if (__syncthreads_or(least < kSplitTiny ? 1 : 0)) {
+        auto check = [&](float x) {
+            const float a = __builtin_fabsf(x);
+            bad |= a > 0.0f && a < kSplitTiny ? 1 : 0;
+        };
+        for (int ch = 0; ch < CH; ++ch)
+            for (int j = 0; j < 8; ++j) check(qrow[16 * ch + j]);
+        for (int k0 = ft.k_lo; k0 < ft.k_hi; k0 += kKBlock) {
+            fetch(k0);
+#pragma unroll
+            for (int i = 0; i < KC; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) check(kst[i][j]);
+#pragma unroll
+            for (int i = 0; i < VC; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (!v_mine(tid + T * i)) break;
+                    check(vst[i][j][0]);
+                    check(vst[i][j][1]);
+                }
+        }
+    }
+    if (__syncthreads_or(bad)) return false;
+
+    if (wave_live && qi < S) {
+        float* orow = ft.out + qi * ft.qw;
+#pragma unroll
+        for (int b = 0; b < MB / 2; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    // dims 64b + 2i, + 1 of rows i = 8g + 4 half + 2u, + 1
+                    const int r = 4 * g + 2 * u;
+                    f32x4 o{acc[2 * b][r], acc[2 * b + 1][r], acc[2 * b][r + 1],
+                            acc[2 * b + 1][r + 1]};
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) o[t] = o[t] / den_all;
+                    *reinterpret_cast<f32x4*>(orow + 64 * b + 16 * g + 8 * half + 4 * u) = o;
+                }
+    }
+    return true;
+}
+
+// At least two waves per SIMD: at most 256 registers a lane.
+template <int HD, int NW, bool PIECES>
+__global__ __launch_bounds__(64 * NW, 2) void flash_attn_kernel(
+    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+    float* __restrict__ out, int64_t S, int64_t H, int64_t KVH, int64_t window, float scale) {
+    static_assert(HD == 64 || HD == 128, "head_dim 64 or 128");
+    constexpr int PLANES = PIECES ? FlashPlanes<HD>::BYTES * (NW == 8 ? 2 : 1) : 0;
+    constexpr int LDS = PLANES > kFp32Lds<HD> ? PLANES : kFp32Lds<HD>;
+    __shared__ __align__(16) unsigned char smem[LDS];
+    const FlashTile ft = flash_tile<HD, NW>(q, k, v, out, S, H, KVH, window);
+    // the running maximum is kept on the unscaled scores: s / scale is
+    // monotone in s, so exp(s/scale - m/scale) = exp2((s - m) * c) with
+    // c = log2(e) / scale, one multiply per weight instead of a division
+    const float c2 = 1.44269504088896340736f / scale;
+    if constexpr (PIECES) {
+        if (flash_pieces<HD, NW>(ft, c2, smem)) return;
+    }
+    flash_fp32<HD, NW>(ft, c2, smem);
+}
+
 }  // namespace
 
 bool launch_flash_attention(const float* q, const float* k, const float* v, float* out,
                             int64_t batch, int64_t seq_len, int64_t q_heads, int64_t kv_heads,
                             int64_t head_dim, int64_t window, hipStream_t s) {
     if (seq_len > INT32_MAX) return false;  // key indices are 32-bit
-    const dim3 grid(static_cast<unsigned>(ceil_div(seq_len, kQTile)),
-                    static_cast<unsigned>(batch * q_heads));
     const float scale = sqrtf(static_cast<float>(head_dim));
+    auto run = [&](auto kernel, int waves) {
+        const dim3 grid(static_cast<unsigned>(ceil_div(seq_len, 32 * waves)),
+                        static_cast<unsigned>(batch * q_heads));
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), 0, s, q, k, v, out, seq_len, q_heads,
+                           kv_heads, window, scale);
+    };
+    // Four waves, two workgroups per CU, or eight waves with two stages of
+    // planes, which stage half as much per wave and meet once per block but
+    // balance the causal tiles less finely (us on MI355X, fp32 MFMA / four / eight
+    // waves: head_dim 64, 512 tiles of 128 queries 54.4 / 48.2 / 52.6, 1,024 tiles
+    // 315 / 224 / 187; head_dim 128, where four waves spill 37 registers, 512 tiles
+    // 167 / 142 / 141, 1,024 tiles 684 / 501 / 378).  Up to 256 tiles of head_dim
+    // 128, at most one workgroup per CU, are bound by one wave's chain through its
+    // key blocks, which the splits lengthen: 81 / 85 / 85 and 46.6 / 51 / 49.8.
+    const int64_t tiles = ceil_div(seq_len, 128) * batch * q_heads;
     switch (head_dim) {
         case 64:
-            hipLaunchKernelGGL(flash_attn_kernel<64>, grid, dim3(256), 0, s, q, k, v, out,
-                               seq_len, q_heads, kv_heads, window, scale);
+            if (tiles >= 1024) run(flash_attn_kernel<64, 8, true>, 8);
+            else run(flash_attn_kernel<64, 4, true>, 4);
             return true;
         case 128:
-            hipLaunchKernelGGL(flash_attn_kernel<128>, grid, dim3(256), 0, s, q, k, v, out,
-                               seq_len, q_heads, kv_heads, window, scale);
+            if (tiles >= 512) run(flash_attn_kernel<128, 8, true>, 8);
+            else run(flash_attn_kernel<128, 4, false>, 4);
             return true;
         default:
             return false;

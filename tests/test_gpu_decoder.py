@@ -83,7 +83,12 @@ ATTN_CASES = [(1, 16, 1, 1, 16, None), (2, 48, 4, 2, 16, None), (2, 48, 4, 2, 16
               (1, 160, 2, 1, 64, None), (1, 160, 2, 1, 64, 130), (2, 272, 3, 3, 32, 20),
               (1, 144, 4, 1, 48, 144), (8, 512, 16, 16, 64, None), (3, 1, 2, 1, 64, None),
               (2, 37, 4, 2, 64, None), (1, 300, 2, 2, 128, None), (2, 200, 4, 1, 128, 50),
-              (1, 129, 16, 4, 128, 33)]
+              (1, 129, 16, 4, 128, 33),
+              # the bf16 pieces' eight waves (512 tiles of 128 queries and more
+              # at head_dim 128, 1,024 at 64): sequences off their 256-query
+              # tiles, grouped heads, windows inside a key block and across them
+              (4, 449, 32, 4, 128, None), (4, 400, 32, 32, 128, 21), (16, 31, 32, 2, 128, None),
+              (8, 385, 32, 4, 64, 300), (16, 129, 32, 8, 64, None)]
 
 
 @pytest.mark.parametrize("B,S,H,KVH,hd,window", ATTN_CASES)
@@ -98,6 +103,39 @@ def test_attention_vs_oracle(ctx, torch, orc, B, S, H, KVH, hd, window):
                   window or 0)
     ref = orc.attention(q, k, v, B, S, H, KVH, hd, window)
     assert_close(host(out), ref, what="attention")
+
+
+@pytest.mark.parametrize("B,S,H,KVH,hd", [(2, 70, 2, 1, 64), (4, 385, 32, 4, 128),
+                                          (8, 385, 32, 4, 64)])
+def test_attention_values_the_pieces_do_not_hold(ctx, torch, orc, B, S, H, KVH, hd):
+    """One tile's infinities, NaN, huge and tiny values leave every other
+    sequence and head as it was, and give what the fp32 loop gives."""
+    rng = np.random.default_rng(hd + S)
+    q = normal(rng, (B * S, H * hd))
+    k = normal(rng, (B * S, KVH * hd))
+    v = normal(rng, (B * S, KVH * hd))
+    v[S // 2, 0] = np.nan                        # sequence 0, key head 0
+    v[S + 5, 1] = np.inf                         # sequence 1: huge values and tiny ones
+    v[S + 9, hd - 1] = 3.4028e38
+    if KVH > 1:
+        v[:, hd:2 * hd] *= np.float32(1e-37)     # key head 1: pieces would keep 8 bits of it
+        k[:, hd:2 * hd] *= np.float32(1e-36)
+        q[:, (H // KVH) * hd:2 * (H // KVH) * hd] *= np.float32(1e36)
+    out = torch.full((B * S, H * hd), 7.0, device="cuda")
+    ctx.attention(dev(torch, q), dev(torch, k), dev(torch, v), out, B, S, H, KVH, hd, 0)
+    got, ref = host(out), orc.attention(q, k, v, B, S, H, KVH, hd, None)
+    # a masked key's infinity or NaN times a zero weight within its key block
+    # is NaN here and skipped in the loop: rows from those keys on, and before
+    # their blocks
+    late = np.arange(B * S) % S >= S // 2
+    rows = (np.arange(B * S) >= 2 * S) | (late & (np.arange(B * S) < S))
+    assert np.array_equal(np.isnan(got[rows]), np.isnan(ref[rows]))
+    for h in range(H):
+        cols = slice(h * hd, (h + 1) * hd)
+        ok = np.isfinite(ref[rows, cols])
+        scale = np.sqrt(np.mean(ref[rows, cols][ok].astype(np.float64) ** 2))
+        diff = np.abs(got[rows, cols][ok].astype(np.float64) - ref[rows, cols][ok])
+        assert np.max(diff) <= 1e-4 * 8 * scale, h
 
 
 def test_attention_after_rope_matches_the_oracle_chain(ctx, torch, orc):
