@@ -171,25 +171,36 @@ __global__ __launch_bounds__(256) void gate_logits_kernel(
 // Small E (up to 8): the ring form.  One wave per workgroup; lane
 // (r, e) = (lane / EB, lane % EB) owns the chain of token t0 + r and expert
 // e.  The R token rows and the EB expert rows stream through an LDS ring of
-// 64-column stages, filled with direct global->LDS buffer loads RING - 1
-// stages ahead (load instruction i of a stage fills 16-byte slot
-// p = 64 i + lane: row p / 16, slot p % 16, which holds the row's chunk
-// (p % 16) ^ (row % 16), so the lanes' reads of one chunk from different
-// rows hit different banks).  Each stage is its own __shared__ array and the
+// 64-column stages, filled with direct global->LDS buffer loads up to RING
+// stages ahead.  Load instruction i of a stage fills 1 KiB with rows 4i ..
+// 4i + 3: chunk q (16 bytes) of row `row` lies at 256 (q / 4) + 64 (row % 4) +
+// 16 (q % 4 ^ row / 4 % 4), so 16 rows' reads of one chunk hit all banks, four
+// lanes load 64 consecutive bytes, and the reads' addresses are one of four
+// per lane plus a constant.  Each stage is its own __shared__ array and the
 // stage loop is unrolled over the ring, so the compiler waits only for the
 // stage being read.  Every lane then runs 64 multiply-adds per stage in
 // column order -- the chain of the kernel above -- with T/R workgroups
 // instead of T/32 (at config 3, 512 instead of 128).
+//
+// Bound: the chain, 4,096 dependent multiply-adds of some 8 cycles.  An XOR of
+// the whole chunk index cost an address addition per read between them, and
+// every stage's reads were waited for before its chain.  Measured on MI355X, us,
+// that form -> this: 7 / 4,096 tokens of d 4096 over 16 experts 31.5 / 36.9 ->
+// 22.5 / 27.7, 4,096 / 16,384 over 8 experts 35.3 / 72.7 -> 24.7 / 54.0, 1,024
+// of d 2048 over 64 experts 20.3 -> 15.1, 4,096 of d 1024 over 8 10.5 -> 8.3.
+// (Four multiply-adds after every pair of reads ran slower, 24.6 us for 22.5:
+// the compiler's own order, a stage's reads and then its chain, stays.)
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kGateRingCols = 64;
 constexpr int kGateRing = 8;
 // Up to this many token x expert logits, 9-64 experts take the per-wave ring
 // with expert blocks (gate_ring_kernel over grid.y); measured on MI355X, us,
 // expert blocks against the workgroup ring / staged kernel: the reference's
-// E = 16 at d 4096, 1 / 64 / 1,024 / 4,096 tokens 39.2 / 38.9 / 40.1 / 43.9
-// against 45.3 / 47.1 / 47.6 / 48.9, at 15,583 tokens 209.9 against 88.8;
-// config 4's E = 64 at d 2048, 16 / 1,024 tokens 23.1 / 25.9 against 86.6 /
-// 91.3, 4,096 86.9 against 88.2, 16,384 352.6 against 105.6.
+// E = 16 at d 4096, 7 / 1,000 / 4,096 tokens 22.5 / 22.7 / 27.7 against 45.3 /
+// 47.6 / 48.9 (a longer grid re-reads the tokens per expert block: with the
+// earlier chain 15,583 tokens took 209.9 against 88.8); config 4's E = 64 at
+// d 2048, 509 / 1,024 tokens 13.3 / 15.1 against 86-91, and with the earlier
+// chain 16,384 352.6 against 105.6.
 constexpr int64_t kGateFewLogits = 65536;
 
 typedef __attribute__((address_space(3))) void gate_lds_t;
@@ -218,10 +229,10 @@ __global__ __launch_bounds__(64) void gate_ring_kernel(
     constexpr int R = 64 / EB;                     // token rows per wave
     constexpr int ROWS = R + EB;                   // staged rows: tokens, then experts
     constexpr int STAGE = ROWS * kGateRingCols;    // floats per stage
-    constexpr int INS = ROWS * 16 / 64;            // load instructions per stage
+    constexpr int INS = ROWS / 4;                  // load instructions per stage
     constexpr int RING = kGateRing;
     static_assert(R % 4 == 0 && EB % 4 == 0, "an instruction's 4 rows come from one matrix");
-    static_assert((RING - 2) * INS <= 63, "vmcnt range");
+    static_assert((RING - 1) * INS <= 63, "vmcnt range");
     __shared__ __align__(16) float r0[STAGE], r1[STAGE], r2[STAGE], r3[STAGE], r4[STAGE],
         r5[STAGE], r6[STAGE], r7[STAGE];
     auto buf = [&](auto u) __attribute__((always_inline)) -> float* {
@@ -242,39 +253,39 @@ __global__ __launch_bounds__(64) void gate_ring_kernel(
     const int64_t nt = T - t0 < R ? T - t0 : R;  // tokens of this wave (>= 1)
     const int64_t e0 = static_cast<int64_t>(blockIdx.y) * EB;  // this wave's expert block
     const int64_t ne = E - e0 < EB ? E - e0 : EB;                // its experts (>= 1)
-    const int64_t nst = (d + kGateRingCols - 1) / kGateRingCols;
+    const int nst = static_cast<int>((d + kGateRingCols - 1) / kGateRingCols);
 
-    // instruction i: rows 4i .. 4i + 3 of the stage, one matrix each
+    // Instruction i fills rows 4i .. 4i + 3 of the stage, one matrix each
     const float* ibase[INS];
     uint32_t ioff[INS];
+    int ichunk[INS];
 #pragma unroll
     for (int i = 0; i < INS; ++i) {
-        const int p = 64 * i + lane, row = p / 16, sl = p % 16;
-        const int chunk = sl ^ (row % 16);
+        const int row = 4 * i + lane / 4 % 4;
+        ichunk[i] = 4 * (lane / 16) + (lane % 4 ^ i % 4);
         if (4 * i < R) {  // token rows
-            const int64_t rr = row < nt ? row : nt - 1;
             ibase[i] = x + t0 * d;
-            ioff[i] = static_cast<uint32_t>((rr * d + 4 * chunk) * 4);
+            ioff[i] = static_cast<uint32_t>((row < nt ? row : nt - 1) * d * 4);
         } else {          // expert rows
-            const int64_t e = row - R < ne ? row - R : ne - 1;
             ibase[i] = w + e0 * d;
-            ioff[i] = static_cast<uint32_t>((e * d + 4 * chunk) * 4);
+            ioff[i] = static_cast<uint32_t>((row - R < ne ? row - R : ne - 1) * d * 4);
         }
     }
-    auto issue = [&](int64_t st, float* dst) __attribute__((always_inline)) {
-        const int64_t j0 = st * kGateRingCols;
+    const int last = static_cast<int>(d) - 4;
+    auto issue = [&](int st, float* dst) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < INS; ++i) {
             // a chunk past the row end loads the row's last chunk (never used)
-            const int chunk = (64 * i + lane) % 16 ^ (((64 * i + lane) / 16) % 16);
-            const int64_t shift = j0 + 4 * chunk <= d - 4 ? j0 : d - 4 - 4 * chunk;
+            const int col = st * kGateRingCols + 4 * ichunk[i];
             gate_load16(ibase[i], (gate_lds_t*)(dst + 256 * i),
-                        static_cast<uint32_t>(ioff[i] + shift * 4));
+                        ioff[i] + static_cast<uint32_t>(col <= last ? col : last) * 4);
         }
     };
-    auto wait_stage = [&](int64_t st) __attribute__((always_inline)) {
-        if (st + RING - 2 < nst) {
-            constexpr int N = (RING - 2) * INS;
+    // Waits until stage st has landed when `ahead` stages may have been issued
+    // after it; near the end fewer were, and it waits for all.
+    auto wait_stage = [&](int st, auto ahead) __attribute__((always_inline)) {
+        if (st + decltype(ahead)::value < nst) {
+            constexpr int N = decltype(ahead)::value * INS;
             __builtin_amdgcn_s_waitcnt(0x3f70 | (N & 15) | ((N >> 4) << 14));
         } else {
             __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0)
@@ -282,56 +293,68 @@ __global__ __launch_bounds__(64) void gate_ring_kernel(
     };
 
     const int r = lane / EB, e = lane % EB;
-    const int xsw = r % 16, wsw = (R + e) % 16;
     float acc = 0.0f;
-    auto consume = [&](const float* stage, int64_t st) __attribute__((always_inline)) {
-        const float* xr = stage + r * kGateRingCols;
-        const float* wr = stage + (R + e) * kGateRingCols;
-        const int64_t j0 = st * kGateRingCols;
-        if (j0 + kGateRingCols <= d) {
-            // the stage's 32 LDS reads first, then the 64-step chain: the
-            // chain no longer waits on a read every 4 steps (bit-identical;
-            // the reference's gate at 1 and 64 tokens 39.6 / 38.6 -> 35.3 /
-            // 34.2 us, config 4's at 64 tokens 24.1 -> 20.7, config 3's 41.3
-            // -> 39.9).  In the workgroup ring below, at four waves per SIMD,
-            // the same 128 registers spilled: 81 -> 428 us at the
-            // reference's 15,583 tokens.
-            f32x4_t xs[16], ws[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                xs[q] = *reinterpret_cast<const f32x4_t*>(xr + 4 * (q ^ xsw));
-                ws[q] = *reinterpret_cast<const f32x4_t*>(wr + 4 * (q ^ wsw));
-            }
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) acc = mac<CONTRACT>(acc, xs[q][c], ws[q][c]);
-        } else {
-            for (int q = 0; q < 16; ++q) {
-                const f32x4_t xv = *reinterpret_cast<const f32x4_t*>(xr + 4 * (q ^ xsw));
-                const f32x4_t wv = *reinterpret_cast<const f32x4_t*>(wr + 4 * (q ^ wsw));
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if (j0 + 4 * q + c < d) acc = mac<CONTRACT>(acc, xv[c], wv[c]);
-            }
-        }
+    // Chunk q of a stage is read GA chunks before the chain reaches it, into
+    // register set q % GA.
+    constexpr int GA = 8;
+    f32x4_t xs[GA], ws[GA];
+    // float offset of chunk c (of 4) of the stage's row `row`
+    auto at = [](int row, int c) __attribute__((always_inline)) {
+        return (row / 4) * 256 + (row % 4) * 16 + 4 * (c ^ row / 4 % 4);
     };
-    gate_static_for(std::make_integer_sequence<int, RING - 1>{}, [&](auto u) __attribute__((always_inline)) {
+    const int xat[4] = {at(r, 0), at(r, 1), at(r, 2), at(r, 3)};
+    const int wat[4] = {at(R + e, 0), at(R + e, 1), at(R + e, 2), at(R + e, 3)};
+    auto chunk_of = [](const float* stage, const int (&at4)[4], int q) __attribute__((always_inline)) {
+        return *reinterpret_cast<const f32x4_t*>(stage + 64 * (q / 4) + at4[q % 4]);
+    };
+    auto read = [&](const float* stage, int q) __attribute__((always_inline)) {
+        xs[q % GA] = chunk_of(stage, xat, q);
+        ws[q % GA] = chunk_of(stage, wat, q);
+    };
+    gate_static_for(std::make_integer_sequence<int, RING>{}, [&](auto u) __attribute__((always_inline)) {
         if (decltype(u)::value < nst) issue(decltype(u)::value, buf(u));
     });
-    for (int64_t st0 = 0; st0 < nst; st0 += RING) {
+    wait_stage(0, std::integral_constant<int, RING - 1>{});
+#pragma unroll
+    for (int q = 0; q < GA; ++q) read(r0, q);
+    const int whole = static_cast<int>(d / kGateRingCols);  // stages without a row end inside
+    for (int st0 = 0; st0 < whole; st0 += RING) {
         gate_static_for(std::make_integer_sequence<int, RING>{}, [&](auto u) __attribute__((always_inline)) {
             constexpr int U = decltype(u)::value;
-            const int64_t st = st0 + U;
-            if (st < nst) {
-                wait_stage(st);
-                consume(buf(u), st);
-                __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this stage is read
-                if (st + RING - 1 < nst)
-                    issue(st + RING - 1, buf(std::integral_constant<int, (U + RING - 1) % RING>{}));
+            const int st = st0 + U;
+            if (st < whole) {
+                const float* next = buf(std::integral_constant<int, (U + 1) % RING>{});
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    if (q == 16 - GA) wait_stage(st + 1, std::integral_constant<int, RING - 2>{});
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+                        acc = mac<CONTRACT>(acc, xs[q % GA][c], ws[q % GA][c]);
+                    // (past the last stage: a stale stage, never used)
+                    if (q + GA < 16) read(buf(u), q + GA);
+                    else read(next, q + GA - 16);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // the chain has consumed this stage's reads: refill it
+                if (st + RING < nst) issue(st + RING, buf(u));
             }
         });
     }
+    if (whole < nst)  // the columns of the last, partial stage
+        gate_static_for(std::make_integer_sequence<int, RING>{}, [&](auto u) __attribute__((always_inline)) {
+            if (whole % RING != decltype(u)::value) return;
+            __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0)
+            const float* stage = buf(u);
+            const int cols = static_cast<int>(d) - whole * kGateRingCols;
+            for (int q = 0; 4 * q < cols; ++q) {
+                const f32x4_t xv = *reinterpret_cast<const f32x4_t*>(stage + 64 * (q / 4) + at(r, q % 4));
+                const f32x4_t wv =
+                    *reinterpret_cast<const f32x4_t*>(stage + 64 * (q / 4) + at(R + e, q % 4));
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (4 * q + c < cols) acc = mac<CONTRACT>(acc, xv[c], wv[c]);
+            }
+        });
     if (r < nt && e < ne) logits[(t0 + r) * E + e0 + e] = acc;
 }
 

@@ -324,6 +324,23 @@ def test_gate_logits_bit_exact(ctx, torch, orc, contract, T, d, E):
 
 
 @pytest.mark.parametrize("contract", [0, 1])
+# the ring kernel's stages of 64 columns, eight of them in flight: one chunk;
+# a row end inside the first stage, on its edge and one chunk past it; seven,
+# eight and nine whole stages, and each with a partial one; one token, a full
+# and a ragged last wave, for 4-expert and 8-expert waves and expert blocks
+@pytest.mark.parametrize("d", [4, 60, 64, 68, 448, 460, 512, 516, 576, 580, 1088])
+@pytest.mark.parametrize("T,E", [(1, 4), (16, 3), (17, 8), (9, 6), (16, 16), (33, 13)])
+def test_gate_ring_stage_edges(ctx, torch, orc, contract, d, T, E):
+    rng = np.random.default_rng(1000 * d + 10 * T + E)
+    x = normal(rng, (T, d))
+    w = normal(rng, (E, d), 0.02)
+    logits = torch.empty((T, E), device="cuda")
+    ctx.gate_logits(dev(torch, x), dev(torch, w), logits, contract=contract)
+    ref = orc.matmul_nt(x, w, contract=contract)
+    assert np.array_equal(host(logits).view(np.int32), ref.view(np.int32))
+
+
+@pytest.mark.parametrize("contract", [0, 1])
 def test_routing_histogram_kat_on_gpu(ctx, torch, orc, contract):
     """The reference's published per-expert row counts
     (docs/microworld/exp-003-moe.html:399-405), recomputed by the GPU gate and
