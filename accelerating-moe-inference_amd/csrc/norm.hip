@@ -11,13 +11,14 @@
 // the same style): inv = 1 / sqrt(sum of x*x / h + eps), y = x * inv * w.
 //
 // The two sums are sequential chains, so one lane owns one row's chain; the
-// work is feeding those chains.  Narrow rows: a workgroup stages R whole
+// work is feeding those chains.  Narrow rows, and wide ones while a single
+// round of workgroups holds them all: a workgroup stages R whole
 // rows in LDS with every thread loading (all of the rows' bytes in flight at
 // once, the only way a latency-bound chain kernel reaches HBM bandwidth),
 // R lanes then run the chains out of LDS, and all threads write y from the
 // staged rows.  x is read once and y written once.  Two 79 KiB workgroups
 // fit a CU (160 KiB of LDS), so one stages while the other runs its chains.
-// Wide rows, of which few fit: the ring kernel (a wave streams its rows'
+// More wide rows, of which few fit: the ring kernel (a wave streams its rows'
 // chains through an LDS ring, many rows per CU in flight) and a 16-byte
 // elementwise pass for y; unaligned wide rows, a register-staged streaming
 // pair.
@@ -59,6 +60,45 @@ __device__ __forceinline__ float normalise(float x, float mean, float inv, float
     return prod + b;
 }
 
+// One row's chain over `h` staged columns, in column order: acc = step(acc, v).
+// Aligned rows read 32 columns ahead of the 32 being added, so that the adds
+// wait on no LDS round trip: 3.6 ns per column on MI355X, the dependent add's
+// own latency, where a round trip per 32 columns and the deviation inside the
+// chain made it 6.6.
+template <bool VEC4, class Step>
+__device__ __forceinline__ float row_chain(const float* row, int64_t h, Step step) {
+    constexpr int AHEAD = 32;
+    float acc = 0.0f;
+    int64_t j = 0;
+    if (VEC4 && h >= 2 * AHEAD) {
+        f32x4 v[2][AHEAD / 4];
+        auto read = [&](int s, int64_t at) {
+#pragma unroll
+            for (int u = 0; u < AHEAD / 4; ++u)
+                v[s][u] = *reinterpret_cast<const f32x4*>(row + at + 4 * u);
+        };
+        auto add = [&](int s) {
+#pragma unroll
+            for (int u = 0; u < AHEAD / 4; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc = step(acc, v[s][u][q]);
+        };
+        read(0, 0);
+        for (; j + 2 * AHEAD <= h; j += 2 * AHEAD) {
+            read(1, j + AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+            add(0);
+            // (past the row's last whole block: columns that are read again below)
+            read(0, j + 3 * AHEAD <= h ? j + 2 * AHEAD : 0);
+            __builtin_amdgcn_sched_barrier(0);
+            add(1);
+        }
+    }
+#pragma unroll 16
+    for (; j < h; ++j) acc = step(acc, row[j]);
+    return acc;
+}
+
 // VEC4: h % 4 == 0 and 16-byte aligned x / y / w / b (16-byte accesses).
 // RMS: no mean (the second chain sums x*x itself), no bias; row_mean unused.
 template <int CONTRACT, bool VEC4, bool RMS>
@@ -75,10 +115,23 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(
     const int64_t n = nr * h;  // the workgroup's rows are one contiguous span of x
     const float* src = x + r0 * h;
 
+    // chunk c of the workgroup's rows: 1,024 columns of row c / cpr (wave-uniform)
+    const int cpr = static_cast<int>((h + 1023) / 1024), nch = nr * cpr;
     if (VEC4) {
-        for (int64_t i = 4 * tid; i < n; i += 4 * 256) {
-            const int64_t r = i / h, j = i - r * h;
-            *reinterpret_cast<f32x4*>(&buf[r * hs + j]) = *reinterpret_cast<const f32x4*>(src + i);
+        for (int c0 = 0; c0 < nch; c0 += 8) {
+            f32x4 v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int c = c0 + u, r = c / cpr;
+                const int64_t j = 1024 * int64_t(c - r * cpr) + 4 * tid;
+                if (c < nch && j < h) v[u] = *reinterpret_cast<const f32x4*>(src + r * h + j);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int c = c0 + u, r = c / cpr;
+                const int64_t j = 1024 * int64_t(c - r * cpr) + 4 * tid;
+                if (c < nch && j < h) *reinterpret_cast<f32x4*>(&buf[r * hs + j]) = v[u];
+            }
         }
     } else {
         for (int64_t i = tid; i < n; i += 256) {
@@ -88,52 +141,37 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(
     }
     __syncthreads();
 
-    if (tid < nr) {
-        // The chains read 32 values ahead (8 16-byte LDS reads issued together),
-        // so each add waits on an LDS round trip once per 32 terms, not per 4.
-        constexpr int kAhead = 32;
-        const float* row = &buf[tid * hs];
-        float sum = 0.0f;
-        int64_t j = RMS ? h : 0;  // RMS: no mean chain
-        if (VEC4)
-            for (; j + kAhead <= h; j += kAhead) {
-                f32x4 v[kAhead / 4];
-#pragma unroll
-                for (int u = 0; u < kAhead / 4; ++u)
-                    v[u] = *reinterpret_cast<const f32x4*>(row + j + 4 * u);
-#pragma unroll
-                for (int u = 0; u < kAhead / 4; ++u)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) sum = sum + v[u][q];
-            }
-#pragma unroll 16
-        for (; j < h; ++j) sum = sum + row[j];
-        const float mean = RMS ? 0.0f : sum / static_cast<float>(h);
-        float var = 0.0f;
-        j = 0;
-        if (VEC4)
-            for (; j + kAhead <= h; j += kAhead) {
-                f32x4 v[kAhead / 4];
-#pragma unroll
-                for (int u = 0; u < kAhead / 4; ++u)
-                    v[u] = *reinterpret_cast<const f32x4*>(row + j + 4 * u);
-#pragma unroll
-                for (int u = 0; u < kAhead / 4; ++u)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float dv = RMS ? v[u][q] : v[u][q] - mean;
-                        var = mac<CONTRACT>(var, dv, dv);
-                    }
-            }
-#pragma unroll 16
-        for (; j < h; ++j) {
-            const float dv = RMS ? row[j] : row[j] - mean;
-            var = mac<CONTRACT>(var, dv, dv);
+    const float* row = &buf[(tid < nr ? tid : 0) * hs];
+    if (!RMS) {
+        if (tid < nr) {
+            const float sum = row_chain<VEC4>(row, h, [](float a, float v) { return a + v; });
+            smean[tid] = sum / static_cast<float>(h);
+            row_mean[r0 + tid] = smean[tid];
         }
+        __syncthreads();
+        // the deviations in the rows' place, by every thread: the second chain
+        // is then one operation per column, and y starts from them
+        for (int r = 0; r < nr; ++r) {
+            const float mean = smean[r];
+            if (VEC4) {
+                for (int64_t j = 4 * tid; j < h; j += 1024) {
+                    f32x4* at = reinterpret_cast<f32x4*>(&buf[r * hs + j]);
+                    f32x4 v = *at;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = v[q] - mean;
+                    *at = v;
+                }
+            } else {
+                for (int64_t j = tid; j < h; j += 256) buf[r * hs + j] = buf[r * hs + j] - mean;
+            }
+        }
+        __syncthreads();
+    }
+    if (tid < nr) {
+        const float var =
+            row_chain<VEC4>(row, h, [](float a, float v) { return mac<CONTRACT>(a, v, v); });
         const float inv = 1.0f / sqrtf(var / static_cast<float>(h) + eps);
-        smean[tid] = mean;
         sinv[tid] = inv;
-        if (!RMS) row_mean[r0 + tid] = mean;
         row_inv[r0 + tid] = inv;
     }
     __syncthreads();
@@ -141,21 +179,24 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(
 
     float* dst = y + r0 * h;
     if (VEC4) {
-        for (int64_t i = 4 * tid; i < n; i += 4 * 256) {
-            const int64_t r = i / h, j = i - r * h;
+#pragma unroll 4
+        for (int c = 0; c < nch; ++c) {
+            const int r = c / cpr;
+            const int64_t j = 1024 * int64_t(c - r * cpr) + 4 * tid;
+            if (j >= h) continue;
             const f32x4 v = *reinterpret_cast<const f32x4*>(&buf[r * hs + j]);
             const f32x4 wv = *reinterpret_cast<const f32x4*>(w + j);
             const f32x4 bv = RMS ? wv : *reinterpret_cast<const f32x4*>(b + j);
             f32x4 o;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                o[q] = normalise<CONTRACT, RMS>(v[q], smean[r], sinv[r], wv[q], bv[q]);
-            *reinterpret_cast<f32x4*>(dst + i) = o;
+                o[q] = normalise<CONTRACT, RMS>(v[q], 0.0f, sinv[r], wv[q], bv[q]);
+            *reinterpret_cast<f32x4*>(dst + r * h + j) = o;
         }
     } else {
         for (int64_t i = tid; i < n; i += 256) {
             const int64_t r = i / h, j = i - r * h;
-            dst[i] = normalise<CONTRACT, RMS>(buf[r * hs + j], smean[r], sinv[r], w[j],
+            dst[i] = normalise<CONTRACT, RMS>(buf[r * hs + j], 0.0f, sinv[r], w[j],
                                               RMS ? 0.0f : b[j]);
         }
     }
@@ -453,7 +494,16 @@ void launch(const float* x, const float* w, const float* b, int64_t rows, int64_
     const int64_t hs = h + kRowPad;
     const bool aligned = h % 4 == 0 && aligned16(x) &&
                          (y == nullptr || (aligned16(y) && aligned16(w) && (RMS || aligned16(b))));
-    if (aligned && kResidentFloats / hs < kRingBelowRows &&
+    // Wide rows that one round of resident workgroups holds stay there too:
+    // every chain runs at once, x is read once and y needs no pass of its own.
+    // Measured on MI355X, us, ring and apply against resident: d = 4096 at 7 /
+    // 512 / 2,048 rows (one round) 55 / 57 / 66 against 37 / 46 / 54, at 4,096
+    // and 15,583 rows (two and eight) 80 / 191 against 99 / 379; d = 2048 at 7 /
+    // 4,096 rows (one) 30 / 42 against 20 / 35, at 8,192 (two) 55 against 68.
+    const int64_t round = hs <= kResidentFloats
+                              ? 2 * static_cast<int64_t>(cus > 0 ? cus : 1) * (kResidentFloats / hs)
+                              : 0;
+    if (rows > round && aligned && kResidentFloats / hs < kRingBelowRows &&
         int64_t(32) * h * 4 < (int64_t(1) << 31)) {
         // rows per wave: enough waves for every CU to hold several (measured
         // on MI355X: 8 rows per wave beat 16 by 1-4 % from 4,096 to 16,384

@@ -1002,6 +1002,29 @@ def test_layer_norm_bit_exact(ctx, torch, orc, contract, rows, h):
 
 
 @pytest.mark.parametrize("contract", [0, 1])
+@pytest.mark.parametrize("rms", [False, True])
+# resident rows: shorter than, exactly and just past the 64 columns of the
+# read-ahead loop, and past 32 more; the 1,024-column load chunks; several rows
+# per workgroup and, on a device of 256 units, the last shape of one round
+# (2,048 rows of 4096, 512 of 20220) and the first that takes the ring
+@pytest.mark.parametrize("rows,h", [(3, 60), (3, 64), (5, 68), (2, 96), (2, 100), (2, 128),
+                                    (700, 1020), (700, 1028), (7, 2052), (2048, 4096),
+                                    (2049, 4096), (512, 20220), (513, 20220)])
+def test_norm_resident_edges(ctx, torch, orc, contract, rms, rows, h):
+    rng = np.random.default_rng(rows + h + contract)
+    x = (2 + 3 * rng.standard_normal((rows, h), dtype=np.float32)).astype(np.float32)
+    w, b = rng.normal(size=(2, h)).astype(np.float32)
+    y = torch.empty((rows, h), device="cuda")
+    if rms:
+        want = orc.rms_norm(x, w, 1e-5, contract)[0]
+        ctx.rms_norm(dev(torch, x), dev(torch, w), y, 1e-5, contract)
+    else:
+        want = orc.layer_norm(x, w, b, 1e-5, contract)[0]
+        ctx.layer_norm(dev(torch, x), dev(torch, w), dev(torch, b), y, 1e-5, contract)
+    assert np.array_equal(host(y), want)
+
+
+@pytest.mark.parametrize("contract", [0, 1])
 @pytest.mark.parametrize("rows,h", [(1, 1), (3, 5), (65, 4096), (130, 33), (4096, 1024),
                                     (3, 30000), (8200, 2600), (2, 30001)])
 def test_rms_norm_bit_exact(ctx, torch, orc, contract, rows, h):
