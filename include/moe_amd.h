@@ -152,7 +152,7 @@ int moe_launch_floor(moe_ctx* ctx, void* stream);
 const char* moe_last_error(void);
 const char* moe_version(void);
 
-/* ---- dense SGEMM, fp32 MFMA.
+/* ---- dense SGEMM, fp32 on the matrix cores (fp32 MFMA, or six products of bf16 pieces).
  * NT: C[M,N] = A[M,K] B[N,K]^T (+ bias[N]); NN: C = A[M,K] B[K,N] (+ bias).
  * Any M, N, K >= 0; K = 0 gives C = bias (or 0).  bias may be NULL. */
 int moe_sgemm_nt(moe_ctx* ctx, const float* A, const float* B,
