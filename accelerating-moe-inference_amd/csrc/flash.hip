@@ -289,14 +289,16 @@ __device__ __forceinline__ void flash_fp32(const FlashTile& ft, float c2, unsign
 // Bound: the waves' own chain, scores -> softmax -> weights -> output; at
 // head_dim 128 a wave's block is 96 MFMAs (3,072 cycles) and about 390 vector
 // instructions (1,560), and two waves share a SIMD.  Measured on MI355X, fp32
-// MFMA -> here: 2 x 2047 queries, 32 heads of 128, 689 -> 383 us (100 -> 179
+// MFMA -> here: 2 x 2047 queries, 32 heads of 128, 689 -> 359 us (100 -> 192
 // TFLOP/s); 4 x 2048, 16 heads, window 512, 366 -> 230; 2 x 2048, 32 heads of
 // 64, 315 -> 187; 8 x 512, 16 heads of 64, 54.4 -> 48.2.  Error against 64 bits
 // 3.1e-7 -> 2.6e-7, 2.9e-7 -> 2.4e-7, 3.0e-7 -> 2.5e-7, 1.8e-7 -> 1.5e-7.  The lagging
-// maximum took the first from 516 to 505 us on four waves, eight waves to 377.
+// maximum took the first from 516 to 505 us on four waves, eight waves to 377, a
+// split without a look for small values to 359.
 //
-// Weights under 2^-100 lose low bits (an error of at most 2^-134 of the
-// largest value); keys, values and queries under it take the fp32 tile.
+// The pieces hold every query, key, value and weight below 2^105 exactly, so
+// the scores and the outputs' sums carry the scale 2^46 (split.hpp): c2 and the
+// last division take it out.
 template <int HD>
 struct FlashPlanes {
     static constexpr int KH = kKBlock * 16 + 16;  // bytes of a K half plane
@@ -311,8 +313,8 @@ struct FlashPlanes {
     }
 };
 
-// Returns whether every value of the tile was split exactly and its sums came
-// out finite; the output is written only then.
+// Returns whether the tile's sums came out finite, every value of it split
+// exactly; the output is written only then.
 template <int HD, int NW>
 __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsigned char* smem) {
     constexpr int T = 64 * NW;
@@ -333,10 +335,6 @@ __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsi
     const int q0 = ft.row0 + 32 * wave, qi = q0 + lq;
     const bool wave_live = q0 < S;
     const int wq_last = q0 + 31 < S ? q0 + 31 : S - 1;
-    float least = 1.0f;  // smallest magnitude this thread has split
-    auto seen = [&](float a, float b) {
-        least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(a)), __builtin_fabsf(b));
-    };
 
     // Q^T operand of chunk ch: dims 16 ch + 8 half .. + 7 of this lane's query
     const float* qrow = ft.q + (qi < S ? qi : S - 1) * ft.qw + 8 * half;
@@ -347,7 +345,6 @@ __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsi
         for (int p = 0; p < 4; ++p) {
             const f32x2 x = *reinterpret_cast<const f32x2*>(qrow + 16 * ch + 2 * p);
             uint32_t w[3];
-            seen(x[0], x[1]);
             split_pair(x[0], x[1], w);
 #pragma unroll
             for (int t = 0; t < 3; ++t) qp[ch][t][p] = w[t];
@@ -380,8 +377,6 @@ __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsi
     };
     auto store4 = [&](const f32x4& x, unsigned char* at, int plane) {
         uint32_t a[3], b[3];
-        seen(x[0], x[1]);
-        seen(x[2], x[3]);
         split_pair(x[0], x[1], a);
         split_pair(x[2], x[3], b);
 #pragma unroll
@@ -444,7 +439,7 @@ __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsi
         }
         const bool full = k0 + kKBlock - 1 <= q0 && (W <= 0 || wq_last - k0 < W);
         float alpha;
-        if (softmax_block<8>(s, full, k0, qi, half, S, W, c2, m_run, den, alpha)) {
+        if (softmax_block<8>(s, full, k0, qi, half, S, W, c2 * kSplitUnscale, m_run, den, alpha)) {
 #pragma unroll
             for (int m = 0; m < MB; ++m)
 #pragma unroll
@@ -473,8 +468,8 @@ __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsi
         }
     }
 
-    // Values the pieces do not hold: non-finite sums, and non-zero magnitudes
-    // below kSplitTiny (zeros split exactly, so a tile that saw less looks again)
+    // What the pieces do not hold: non-finite sums, and queries whose scores all
+    // passed the range (every query sees a key, so a sum of weights is above 0)
     const float den_all = den + __shfl_xor(den, 32, 64);
     int bad = 0;
     if (wave_live && qi < S) {
@@ -483,34 +478,12 @@ __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsi
         for (int m = 0; m < MB; ++m)
 #pragma unroll
             for (int r = 0; r < 16; ++r) z = fmaf(acc[m][r], 0.0f, z);
-        bad = !(z == 0.0f);
-    }
-    if (__syncthreads_or(least < kSplitTiny ? 1 : 0)) {
-        auto check = [&](float x) {
-            const float a = __builtin_fabsf(x);
-            bad |= a > 0.0f && a < kSplitTiny ? 1 : 0;
-        };
-        for (int ch = 0; ch < CH; ++ch)
-            for (int j = 0; j < 8; ++j) check(qrow[16 * ch + j]);
-        for (int k0 = ft.k_lo; k0 < ft.k_hi; k0 += kKBlock) {
-            fetch(k0);
-#pragma unroll
-            for (int i = 0; i < KC; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) check(kst[i][j]);
-#pragma unroll
-            for (int i = 0; i < VC; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (!v_mine(tid + T * i)) break;
-                    check(vst[i][j][0]);
-                    check(vst[i][j][1]);
-                }
-        }
+        bad = !(z == 0.0f && den_all > 0.0f);
     }
     if (__syncthreads_or(bad)) return false;
 
     if (wave_live && qi < S) {
+        const float den_s = den_all / kSplitUnscale;
         float* orow = ft.out + qi * ft.qw;
 #pragma unroll
         for (int b = 0; b < MB / 2; ++b)
@@ -523,7 +496,7 @@ __device__ __forceinline__ bool flash_pieces(const FlashTile& ft, float c2, unsi
                     f32x4 o{acc[2 * b][r], acc[2 * b + 1][r], acc[2 * b][r + 1],
                             acc[2 * b + 1][r + 1]};
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) o[t] = o[t] / den_all;
+                    for (int t = 0; t < 4; ++t) o[t] = o[t] / den_s;
                     *reinterpret_cast<f32x4*>(orow + 64 * b + 16 * g + 8 * half + 4 * u) = o;
                 }
     }

@@ -1362,8 +1362,11 @@ __device__ __forceinline__ void direct_tile(const GemmArgs& p, int mt, int nt, i
 // reads stage kt % 2, splits the rows of step kt + 1 (loaded during step
 // kt - 1) into the other one and starts the loads of step kt + 2; one barrier
 // per step.  The split runs once per workgroup, not once per wave that reads
-// a row: 168 vector instructions per wave and step, which issue under its 48
-// MFMAs.
+// a row: about 180 vector instructions per wave and step, which issue under its
+// 48 MFMAs.  (A scaled split needs no look at the values: with the smallest
+// magnitude tracked beside it, and tiles that saw a zero reading their operands
+// again, 1000 x 3001 x 777 took 67 us for 46, 4096^3 805 for 652, config 3's layer
+// 15.6 ms for 14.4, and a tenth of zero rows cost 5-11 % more.)
 //
 // Bound: power.  The bare MFMA loop holds about 1,750 TFLOP/s of bf16 on this
 // card at 1.7 GHz; in these tiles the matrix pipe is busy 64-74 % of the cycles
@@ -1403,7 +1406,7 @@ constexpr int split_prefetch = NB * C::FM * C::FN <= 4 ? 2 : 1;
 
 // One 32x32 block over K columns [0, K) of the fp32 rows at `a` and `b` (this
 // lane's row lane % 32 of the block's A and B rows; b's elements bstep floats
-// apart) on fp32 MFMA: blocks whose split is not exact.  ANY: any K and any
+// apart) on fp32 MFMA: blocks of values or sums that the pieces do not hold.  ANY: any K and any
 // alignment, columns past K count 0.
 template <bool NN, bool ANY>
 __device__ __attribute__((noinline)) f32x16 fp32_block(const float* a, const float* b,
@@ -1574,14 +1577,11 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
             st[i][j] = __float_as_uint(k < K ? row[k] : 0.0f);
         }
     };
-    float least = 1.0f;  // smallest magnitude this thread has split
     // the pieces of four consecutive k of an operand's row, to `at` + 8 bytes per piece plane
     auto split4 = [&](const u32x4& raw, unsigned char* at, int plane) {
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(raw[j]);
-        least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(v[0])), __builtin_fabsf(v[1]));
-        least = __builtin_fminf(__builtin_fminf(least, __builtin_fabsf(v[2])), __builtin_fabsf(v[3]));
         uint32_t lo[3], hi[3];
         split_pair(v[0], v[1], lo);
         split_pair(v[2], v[3], hi);
@@ -1720,34 +1720,7 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
     else if (live == 1) k_loop(std::integral_constant<int, 1>{});
     else k_loop(std::integral_constant<int, 0>{});
 
-    // Tiles that saw a magnitude below kSplitTiny look whether it was only
-    // zeros (which split exactly); a non-zero one takes the fp32 path.
-    int tiny = 0;
-    if (__syncthreads_or(least < kSplitTiny ? 1 : 0)) {
-        for (int kt = 0; kt < nk; ++kt) {
-#pragma unroll
-            for (int i = 0; i < CH; ++i) load_chunk(0, i, k_bytes(kt, 1), k_bytes(kt, bstep));
-#pragma unroll
-            for (int i = 0; i < CH + (NN ? 1 : 0); ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float v = __builtin_fabsf(__uint_as_float(stages[0][i][j]));
-                    tiny |= v > 0.0f && v < kSplitTiny ? 1 : 0;
-                }
-        }
-        if (ANY && ktail < K) {
-#pragma unroll
-            for (int i = 0; i < CH; ++i) load_tail(i);
-#pragma unroll
-            for (int i = 0; i < CH + (NN ? 1 : 0); ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float v = __builtin_fabsf(__uint_as_float(stages[0][i][j]));
-                    tiny |= v > 0.0f && v < kSplitTiny ? 1 : 0;
-                }
-        }
-        tiny = __syncthreads_or(tiny);
-    }
+    // Blocks with a value or a sum that the pieces do not hold: fp32 MFMA
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -1757,10 +1730,14 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
                 float z = 0.0f;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) z = __builtin_fmaf(acc[nb][bi][bj][r], 0.0f, z);
-                if (bi < live && (tiny || __any(!(z == 0.0f))))
+                if (bi < live && __any(!(z == 0.0f))) {
                     acc[nb][bi][bj] = fp32_block<NN, ANY>(
                         a_row(arow0 + bi * 32 + lr) + kbeg,
                         b_row(nb, bcol0 + bj * 32 + lr) + kbeg * bstep, bstep, K - kbeg);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[nb][bi][bj][r] *= kSplitUnscale;
+                }
             }
     if constexpr (NN) {
         // two adjacent columns per lane and row: one 8-byte store where both

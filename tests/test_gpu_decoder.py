@@ -138,6 +138,40 @@ def test_attention_values_the_pieces_do_not_hold(ctx, torch, orc, B, S, H, KVH, 
         assert np.max(diff) <= 1e-4 * 8 * scale, h
 
 
+@pytest.mark.parametrize("B,S,H,KVH,hd,gap", [
+    (1, 70, 2, 1, 64, 122), (8, 385, 32, 4, 64, 118), (4, 385, 32, 4, 128, 124),
+    (2, 70, 2, 1, 128, 120)])
+def test_attention_small_weights_keep_their_bits(ctx, torch, B, S, H, KVH, hd, gap):
+    """The first key dominates and its value is zero, so the outputs are the
+    other keys' values under weights of about 2^-gap.  The scores are exact here
+    (two non-zero columns of few bits).  A weight's exponent, up to 128 and so
+    rounded by at most 2^-18, and the logarithm's constant in it, another 2^-18, leave
+    a relative error of 2^-17 ln 2 = 5.3e-6; the sums and the quotient some 1e-6."""
+    rng = np.random.default_rng(S + hd + gap)
+    scale = np.sqrt(hd)
+    q = np.zeros((B, S, H, hd), np.float32)
+    k = np.zeros((B, S, KVH, hd), np.float32)
+    v = rng.uniform(0.5, 1.5, (B, S, KVH, hd)).astype(np.float32)
+    q[..., 0], q[..., 1] = 16.0, 1.0
+    # the first key's exponent is above the others' by gap, an exact score
+    k[:, 0, :, 0] = np.round(gap * scale / 1.4426950408889634 / 16 * 256) / 256
+    k[:, 1:, :, 1] = np.round(rng.uniform(-1, 1, (B, S - 1, KVH)) * 256) / 256
+    v[:, 0] = 0.0
+    out = torch.empty((B * S, H * hd), device="cuda")
+    ctx.attention(dev(torch, q.reshape(B * S, -1)), dev(torch, k.reshape(B * S, -1)),
+                  dev(torch, v.reshape(B * S, -1)), out, B, S, H, KVH, hd, 0)
+    got = host(out).reshape(B, S, H, hd)
+    for h in range(H):
+        s = np.einsum("bik,bjk->bij", q[:, :, h].astype(np.float64),
+                      k[:, :, h // (H // KVH)].astype(np.float64)) / scale
+        s = np.where(np.tril(np.ones((S, S), bool)), s, -np.inf)
+        w = np.exp(s - s.max(axis=2, keepdims=True))
+        ref = (w / w.sum(axis=2, keepdims=True)) @ v[:, :, h // (H // KVH)].astype(np.float64)
+        assert np.all(got[:, 0, h] == 0)
+        rel = np.abs(got[:, 1:, h] / ref[:, 1:] - 1)
+        assert np.max(rel) <= 8e-6, (h, np.max(rel))
+
+
 def test_attention_after_rope_matches_the_oracle_chain(ctx, torch, orc):
     # the order the decoder runs them in: RoPE on q, k, then attention
     rng = np.random.default_rng(21)

@@ -714,6 +714,82 @@ def test_sgemm_bf16_pieces_special_values(ctx, torch, orc, layout, N, K):
     assert abs(got[100, 5] - exact[100, 5]) <= 2.0 ** -22 * K * big
 
 
+@pytest.mark.parametrize("layout,N,K", [("nt", 129, 70), ("nt", 300, 777), ("nn", 131, 37)])
+def test_sgemm_one_value_leaves_the_other_rows(ctx, torch, layout, N, K):
+    """A tiny value, a denormal or a zero in one row of A: every other row of
+    the product keeps every bit."""
+    rng = np.random.default_rng(N + K)
+    M = 200
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = dev(torch, rng.standard_normal((N, K) if layout == "nt" else (K, N)).astype(np.float32))
+
+    def product(value):
+        aa = a.copy()
+        aa[70, 3] = value
+        c = torch.empty((M, N), device="cuda")
+        (ctx.sgemm_nt if layout == "nt" else ctx.sgemm_nn)(dev(torch, aa), b, c)
+        return host(c)
+
+    others = np.arange(M) != 70
+    ref = product(1.0)[others]
+    for value in (1e-35, 1e-42, 0.0):
+        assert np.array_equal(product(value)[others].view(np.int32), ref.view(np.int32)), value
+
+
+@pytest.mark.parametrize("act", [0, 1])
+def test_expert_ffn_one_value_leaves_the_other_tokens(ctx, torch, orc, act):
+    """A tiny value in one token: the other tokens' rows keep every bit."""
+    rng = np.random.default_rng(act + 50)
+    T, d, E, k, d_ff = 300, 64, 2, 1, 160
+    x, w1, w3, w2, topk = _ffn_case(rng, T, d, E, k, d_ff, act)
+    roff, rperm, _ = orc.permute(topk, E)
+    w = [None if t is None else dev(torch, t) for t in (w1, w3, w2)]
+
+    def run(value):
+        xx = x.copy()
+        xx[70, 3] = value
+        h = torch.empty((T * k, d_ff), device="cuda")
+        out = torch.empty((T * k, d), device="cuda")
+        ctx.expert_ffn_grouped(dev(torch, xx), dev(torch, rperm), dev(torch, roff), *w, k, h, out,
+                               act=act)
+        return host(out)
+
+    others = rperm != 70
+    ref = run(1.0)[others]
+    for value in (1e-35, 1e-42, 0.0):
+        assert np.array_equal(run(value)[others].view(np.int32), ref.view(np.int32)), value
+
+
+@pytest.mark.parametrize("layout,N,K", [("nt", 301, 70), ("nn", 301, 70), ("nt", 320, 1024),
+                                        ("nn", 320, 1024)])
+def test_sgemm_every_magnitude(ctx, torch, layout, N, K):
+    """Rows of A and columns of B from fp32's smallest denormals to its largest
+    values: every sum that fits fp32 to the rounding of its products, 2^-24 each
+    and what the pieces leave out of them, 2^-24 more, and of the 6 K / 16
+    additions, 2^-23 each however the matrix unit rounds."""
+    rng = np.random.default_rng(N + K)
+    M = 1100
+    ea = rng.integers(-148, 126, M)
+    eb = rng.integers(-148, 126, N)
+    with np.errstate(over="ignore", under="ignore"):
+        a = np.ldexp(rng.uniform(-1, 1, (M, K)), ea[:, None]).astype(np.float32)
+        b = np.ldexp(rng.uniform(-1, 1, (N, K)), eb[:, None]).astype(np.float32)
+    c = torch.empty((M, N), device="cuda")
+    if layout == "nt":
+        ctx.sgemm_nt(dev(torch, a), dev(torch, b), c)
+    else:
+        ctx.sgemm_nn(dev(torch, a), dev(torch, np.ascontiguousarray(b.T)), c)
+    got = host(c).astype(np.float64)
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    mag = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T
+    fits = mag < 2.0 ** 127
+    assert fits.mean() > 0.5
+    bound = (6 * K / 16 + 2) * 2.0 ** -23 * mag + K * 2.0 ** -149
+    with np.errstate(invalid="ignore"):
+        diff = np.abs(got - exact)
+    assert np.all(diff[fits] <= bound[fits])
+
+
 # Shapes the planner sends to the grouped skinny kernel (few rows per expert,
 # K a multiple of 16; the context's default tile dealing): config 1's experts
 # (32-row workgroups, SiLU), a decoder's last rows (8 tokens, 16-row
