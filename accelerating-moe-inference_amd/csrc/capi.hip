@@ -211,8 +211,14 @@ DensePlan plan_dense(moe_ctx* ctx, bool nn, bool direct, int64_t M, int64_t N, i
     if (!direct) {
         // unaligned rows or a ragged K: the pieces take them, the fp32 tiles
         // do not (only the register-staged 128 x 128 kernel does, and where
-        // the pieces' offsets pass 2 GiB, or NN has one column, still runs)
-        return moe::pieces_fit(nn, M, N, K) ? plan_pieces(ctx, M, N, K, false).plan : best;
+        // the pieces' offsets pass 2 GiB, or NN has one column, still runs).
+        // So do sums of one or two products: what the pieces leave out of a
+        // product is as large as its rounding, and their fewer additions make
+        // up for it from three products on (error against 64 bits, 2-norm,
+        // fp32 MFMA / pieces at K = 1, 2, 3, 4: 2.5 / 3.4, 3.1 / 3.4, 3.6 / 3.3,
+        // 4.0 / 3.2 e-8; largest, in 2^-24 of the products' magnitudes, 1.0 /
+        // 2.5, 1.9 / 2.8, 2.5 / 2.2, 3.0 / 2.1).
+        return K > 2 && moe::pieces_fit(nn, M, N, K) ? plan_pieces(ctx, M, N, K, false).plan : best;
     }
     static const int env_tile = env_int("MOE_DENSE_TILE", -1);
     static const int env_splits = env_int("MOE_DENSE_SPLITS", 0);

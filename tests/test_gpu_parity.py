@@ -760,6 +760,29 @@ def test_expert_ffn_one_value_leaves_the_other_tokens(ctx, torch, orc, act):
         assert np.array_equal(run(value)[others].view(np.int32), ref.view(np.int32)), value
 
 
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("M,N", [(5, 7), (300, 130), (1000, 515)])
+@pytest.mark.parametrize("K", [1, 2])
+def test_sgemm_one_and_two_products(ctx, torch, layout, M, N, K):
+    """A single product is the fp32 product, rounded once; a sum of two is
+    rounded at most twice, 2^-24 each."""
+    rng = np.random.default_rng(M + K)
+    a = rng.standard_normal((M, K)).astype(np.float32)
+    b = rng.standard_normal((N, K)).astype(np.float32)
+    c = torch.empty((M, N), device="cuda")
+    if layout == "nt":
+        ctx.sgemm_nt(dev(torch, a), dev(torch, b), c)
+    else:
+        ctx.sgemm_nn(dev(torch, a), dev(torch, np.ascontiguousarray(b.T)), c)
+    got = host(c)
+    if K == 1:
+        assert np.array_equal(got, a * b.T)
+        return
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    mag = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T
+    assert np.all(np.abs(got - exact) <= 2.0 ** -23 * (1 + 2.0 ** -20) * mag)
+
+
 @pytest.mark.parametrize("layout,N,K", [("nt", 301, 70), ("nn", 301, 70), ("nt", 320, 1024),
                                         ("nn", 320, 1024)])
 def test_sgemm_every_magnitude(ctx, torch, layout, N, K):
