@@ -63,8 +63,7 @@ __device__ __forceinline__ float normalise(float x, float mean, float inv, float
 // One row's chain over `h` staged columns, in column order: acc = step(acc, v).
 // Aligned rows read 32 columns ahead of the 32 being added, so that the adds
 // wait on no LDS round trip: 3.6 ns per column on MI355X, the dependent add's
-// own latency, where a round trip per 32 columns and the deviation inside the
-// chain made it 6.6.
+// own latency.
 template <bool VEC4, class Step>
 __device__ __forceinline__ float row_chain(const float* row, int64_t h, Step step) {
     constexpr int AHEAD = 32;
@@ -112,32 +111,52 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(
     const int64_t r0 = static_cast<int64_t>(blockIdx.x) * R;
     const int nr = static_cast<int>(rows - r0 < R ? rows - r0 : R);
     const int64_t hs = h + kRowPad;
-    const int64_t n = nr * h;  // the workgroup's rows are one contiguous span of x
+    const int n = static_cast<int>(nr * h);  // the workgroup's rows are one contiguous span of x
     const float* src = x + r0 * h;
+    // Every pass over the rows deals the span's columns (VEC4: groups of four)
+    // to the threads in turn, whatever h: thread tid's first one, and from one
+    // to its next 256 further on, as (row, column).  Column i lies at i + row *
+    // kRowPad.  (Row by row in chunks of 1,024 columns, which leaves threads idle
+    // past the end of each row, layer norms of 37,181 x 12 / 24,334 x 108 / 32,768 x
+    // 512 / 15,583 x 1028 / 15,583 x 1024 took 57 / 28 / 62 / 66 / 48 us; dealt this
+    // way 9 / 9 / 36 / 43 / 42.)
+    constexpr int G = VEC4 ? 4 : 1;
+    const int hh = static_cast<int>(h), step_r = G * 256 / hh, step_j = G * 256 % hh;
+    auto columns = [&](auto&& body) {
+        int r = G * tid / hh, j = G * tid % hh;
+        for (int i = G * tid; i < n; i += G * 256) {
+            body(i, r, j);
+            r += step_r;
+            j += step_j;
+            if (j >= hh) {
+                j -= hh;
+                ++r;
+            }
+        }
+    };
 
-    // chunk c of the workgroup's rows: 1,024 columns of row c / cpr (wave-uniform)
-    const int cpr = static_cast<int>((h + 1023) / 1024), nch = nr * cpr;
     if (VEC4) {
-        for (int c0 = 0; c0 < nch; c0 += 8) {
+        // eight loads in flight per thread
+        int r = G * tid / hh, j = G * tid % hh;
+        for (int i0 = G * tid; i0 < n; i0 += 8 * G * 256) {
             f32x4 v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int c = c0 + u, r = c / cpr;
-                const int64_t j = 1024 * int64_t(c - r * cpr) + 4 * tid;
-                if (c < nch && j < h) v[u] = *reinterpret_cast<const f32x4*>(src + r * h + j);
-            }
+            for (int u = 0; u < 8; ++u)
+                if (i0 + u * G * 256 < n) v[u] = *reinterpret_cast<const f32x4*>(src + i0 + u * G * 256);
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                const int c = c0 + u, r = c / cpr;
-                const int64_t j = 1024 * int64_t(c - r * cpr) + 4 * tid;
-                if (c < nch && j < h) *reinterpret_cast<f32x4*>(&buf[r * hs + j]) = v[u];
+                const int i = i0 + u * G * 256;
+                if (i < n) *reinterpret_cast<f32x4*>(&buf[i + r * kRowPad]) = v[u];
+                r += step_r;
+                j += step_j;
+                if (j >= hh) {
+                    j -= hh;
+                    ++r;
+                }
             }
         }
     } else {
-        for (int64_t i = tid; i < n; i += 256) {
-            const int64_t r = i / h, j = i - r * h;
-            buf[r * hs + j] = src[i];
-        }
+        columns([&](int i, int r, int) { buf[i + r * kRowPad] = src[i]; });
     }
     __syncthreads();
 
@@ -151,20 +170,18 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(
         __syncthreads();
         // the deviations in the rows' place, by every thread: the second chain
         // is then one operation per column, and y starts from them
-        for (int r = 0; r < nr; ++r) {
-            const float mean = smean[r];
-            if (VEC4) {
-                for (int64_t j = 4 * tid; j < h; j += 1024) {
-                    f32x4* at = reinterpret_cast<f32x4*>(&buf[r * hs + j]);
-                    f32x4 v = *at;
+        columns([&](int i, int r, int) {
+            if constexpr (VEC4) {
+                f32x4* at = reinterpret_cast<f32x4*>(&buf[i + r * kRowPad]);
+                f32x4 v = *at;
+                const float mean = smean[r];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) v[q] = v[q] - mean;
-                    *at = v;
-                }
+                for (int q = 0; q < 4; ++q) v[q] = v[q] - mean;
+                *at = v;
             } else {
-                for (int64_t j = tid; j < h; j += 256) buf[r * hs + j] = buf[r * hs + j] - mean;
+                buf[i + r * kRowPad] = buf[i + r * kRowPad] - smean[r];
             }
-        }
+        });
         __syncthreads();
     }
     if (tid < nr) {
@@ -178,28 +195,21 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(
     if (y == nullptr) return;
 
     float* dst = y + r0 * h;
-    if (VEC4) {
-#pragma unroll 4
-        for (int c = 0; c < nch; ++c) {
-            const int r = c / cpr;
-            const int64_t j = 1024 * int64_t(c - r * cpr) + 4 * tid;
-            if (j >= h) continue;
-            const f32x4 v = *reinterpret_cast<const f32x4*>(&buf[r * hs + j]);
+    columns([&](int i, int r, int j) {
+        if constexpr (VEC4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(&buf[i + r * kRowPad]);
             const f32x4 wv = *reinterpret_cast<const f32x4*>(w + j);
             const f32x4 bv = RMS ? wv : *reinterpret_cast<const f32x4*>(b + j);
             f32x4 o;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
                 o[q] = normalise<CONTRACT, RMS>(v[q], 0.0f, sinv[r], wv[q], bv[q]);
-            *reinterpret_cast<f32x4*>(dst + r * h + j) = o;
-        }
-    } else {
-        for (int64_t i = tid; i < n; i += 256) {
-            const int64_t r = i / h, j = i - r * h;
-            dst[i] = normalise<CONTRACT, RMS>(buf[r * hs + j], 0.0f, sinv[r], w[j],
+            *reinterpret_cast<f32x4*>(dst + i) = o;
+        } else {
+            dst[i] = normalise<CONTRACT, RMS>(buf[i + r * kRowPad], 0.0f, sinv[r], w[j],
                                               RMS ? 0.0f : b[j]);
         }
-    }
+    });
 }
 
 // ---- rows wider than kResidentFloats - kRowPad: streaming statistics.  One

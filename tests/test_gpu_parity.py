@@ -1123,6 +1123,47 @@ def test_norm_resident_edges(ctx, torch, orc, contract, rms, rows, h):
     assert np.array_equal(host(y), want)
 
 
+# columns dealt to 256 threads in turn, four at a time where rows are aligned:
+# several rows per turn, a row end inside a turn, exactly one turn per row, one
+# and a bit; more rows than a workgroup holds
+@pytest.mark.parametrize("contract", [0, 1])
+@pytest.mark.parametrize("rows,h", [(33000, 4), (33001, 12), (700, 252), (1500, 255), (1500, 256),
+                                    (1500, 257), (2100, 1016), (1100, 1024), (1100, 1027)])
+def test_norm_narrow_rows(ctx, torch, orc, contract, rows, h):
+    rng = np.random.default_rng(rows + h + contract)
+    x = (1 + rng.standard_normal((rows, h), dtype=np.float32)).astype(np.float32)
+    w, b = rng.normal(size=(2, h)).astype(np.float32)
+    y = dev(torch, x)
+    ctx.layer_norm(y, dev(torch, w), dev(torch, b), y, 1e-5, contract)
+    assert np.array_equal(host(y), orc.layer_norm(x, w, b, 1e-5, contract)[0])
+    y = dev(torch, x)
+    ctx.rms_norm(y, dev(torch, w), y, 1e-5, contract)
+    assert np.array_equal(host(y), orc.rms_norm(x, w, 1e-5, contract)[0])
+
+
+def test_norm_of_narrow_rows_costs_no_more(ctx, torch):
+    """1 M values in rows of 12, 32 and 108 against rows of 512: the chains are
+    shorter and the bytes the same, so twice the time is too much (rows dealt to
+    1,024-column chunks took 3 to 6 times)."""
+    def us(rows, h):
+        x, y = (torch.ones((rows, h), device="cuda") for _ in range(2))
+        w, b = (torch.ones(h, device="cuda") for _ in range(2))
+        best = float("inf")
+        for _ in range(8):
+            beg, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            beg.record()
+            for _ in range(20):
+                ctx.layer_norm(x, w, b, y)
+            end.record()
+            end.synchronize()
+            best = min(best, beg.elapsed_time(end) * 50)
+        return best
+
+    wide = us(2048, 512)
+    for h in (12, 32, 108):
+        assert us((1 << 20) // h, h) <= 2 * wide, h
+
+
 @pytest.mark.parametrize("contract", [0, 1])
 @pytest.mark.parametrize("rows,h", [(1, 1), (3, 5), (65, 4096), (130, 33), (4096, 1024),
                                     (3, 30000), (8200, 2600), (2, 30001)])
