@@ -2578,6 +2578,13 @@ void launch_gemm(const GemmArgs& args, bool nn, bool grouped, int epi, bool vec,
     // its 4,096 / 1,024 / 509 tokens 2.15 / 0.774 / 0.622 -> 2.03 / 0.702 / 0.530; the
     // reference's 7 n-tiles 1.31 -> 1.33)
     if (env_group == 0 && grouped && epi != EPI_STORE && !a.fp32 && a.n_tiles >= 8) group = 0;
+    // ... and on fp32 MFMA over many experts while they average at most 32 rows (same box, us
+    // per w1/w3 launch, groups of 8 -> m-fastest: config 4's experts at top-1 of 256 tokens 151
+    // -> 127; 128 experts of 1024 x 1024 at top-2 of 128 / 256 tokens 61 / 79 -> 56 / 73; ragged
+    // widths, 64 experts of 2040 x 1400 and 32 of 1000 x 2000, level)
+    if (env_group == 0 && grouped && epi != EPI_STORE && a.fp32 && a.E >= 32 &&
+        a.rows_limit <= 32 * int64_t(a.E))
+        group = 0;
     if (group < 1 || group > a.m_tiles) group = a.m_tiles;
     a.group_m = group;
     if (a.k_splits <= 1) {
