@@ -423,16 +423,17 @@ struct FfnPlan {
     bool fp32 = false;      // the tiles on fp32 MFMA (GemmArgs::fp32): few_rows, ragged K
 };
 
-// Layers whose experts hold few rows, at most 4 on average, or 16 with up to
-// 16 experts: they are bound by reading the weights, and the fp32 MFMA tiles,
-// whose loads run two K steps ahead, read them faster than the bf16 pieces,
-// whose loads run one ahead (same box, us, w1/w3 and w2: config 3 at 4 / 24
-// / 64 tokens fp32 566 / 938 / 924 and 280 / 413 / 435, pieces 750 / 1,003 /
-// 1,024 and 379 / 562 / 568; at 128 tokens, 32 rows each, 1,219 and 757
-// against 1,076 and 591.  Config 4's 64 experts, unevenly loaded, at 16 / 32
-// tokens 170 / 210 against 200 / 241; at 64 / 128 tokens, 8 and 16 rows each,
-// 342 / 395 against 275 / 304).
-bool few_rows(int64_t pairs, int64_t E) { return pairs <= 4 * E || (E <= 16 && pairs <= 16 * E); }
+// Layers whose experts hold at most 2 rows on average, or 4 with more than 16
+// experts: bound by reading the weights, which both kinds of tile do about as
+// fast, and the fp32 tiles' stream-K deals evenly where few experts hold rows at
+// all.  With more rows the pieces are level or faster.  Same box, us, w1/w3 + w2,
+// fp32 MFMA / pieces: under a Zipf bias 8 experts of config 3 at top-1 of 16 / 24
+// tokens (2 / 3 rows) 827 / 994, 698 / 605, config 4's 64 at top-1 of 192 / 384 tokens
+// (3 / 6) 150 / 203, 208 / 206, 128 of 1024 x 1024 at top-2 of 192 / 512 (3 / 8) 91 /
+// 99, 128 / 107; evenly loaded config 3 at 3 / 6 / 16 rows 1,229 / 1,077, 1,303 / 1,178,
+// 1,328 / 1,184, 16 experts of 2048 x 4096 at 3 / 6 / 16 437 / 393, 429 / 398, 420 / 399,
+// 24 of 2048 x 4096 at 2 / 4 / 8 555 / 581, 632 / 606, 624 / 610.
+bool few_rows(int64_t pairs, int64_t E) { return pairs <= (E > 16 ? 4 : 2) * E; }
 
 int grouped_slots(moe_ctx* ctx, moe::GemmUse use, bool fp32, bool sk) {
     int& occ = (sk ? ctx->sk_blocks_per_cu : ctx->grouped_blocks_per_cu)[fp32 ? 1 : 0]
@@ -504,7 +505,11 @@ int64_t expected_m_tiles(int64_t pairs, int64_t E, int bm) {
 // one tile per workgroup / stream-K: the reference's layer at 256 / 1,024 /
 // 4,096 tokens, fill 0.1 / 0.2 / 0.5, 387 / 405 / 548 against 120 / 170 / 454;
 // config 5 at 256 tokens, 0.3, 108 against 98; at 1,024, 0.9, 184 against 211;
-// config 3 at 256 / 4,096 tokens 1,210 / 11,101 against 1,348 / 11,505), w2
+// config 3 at 256 / 4,096 tokens 1,210 / 11,101 against 1,348 / 11,505).  From
+// 0.7 to 1.0 it depends on the load, which the host does not know: config 4's
+// experts at top-1 of 512 / 1,024 tokens 381 / 393 against 343 / 354, at top-8 of
+// 64 / 96 under the Zipf bias 212 / 234 against 242 / 294, and short K loops lose
+// (K 256, 116 against 142; K 96, 85 against 103).  w2
 // takes its K splits instead (config 3 4,820 + 129 us of combine against 6,315
 // + 39; 1,024 tokens 1,519 + 39 against 2,029 + 13; config 5 at 256 / 1,024
 // tokens 53 / 96 against 58 / 107; the reference's at 1,024 tokens level).

@@ -578,6 +578,25 @@ def test_expert_ffn_bf16_pieces(ctx, torch, T, d, E, k, d_ff, act):
     assert err <= 8 * 2.0 ** -23 * np.sqrt(6 * max(d, d_ff, 16) / 16)
 
 
+# Few rows per expert, about the lines between the fp32 tiles and the pieces (two
+# rows on average up to 16 experts, four with more), evenly and unevenly loaded.
+@pytest.mark.parametrize("T,d,E,k,d_ff,skew", [
+    (128, 512, 64, 2, 1408, False), (129, 512, 64, 2, 1408, False), (300, 512, 64, 1, 1408, True),
+    (384, 512, 64, 1, 1024, False), (150, 256, 64, 4, 2048, True), (16, 1024, 16, 2, 4096, False),
+    (17, 1024, 16, 2, 4096, False), (9, 1024, 8, 2, 4096, True), (130, 256, 16, 2, 4096, False),
+])
+def test_expert_ffn_few_rows(ctx, torch, orc, T, d, E, k, d_ff, skew):
+    rng = np.random.default_rng(T + d + E + k)
+    x, w1, w3, w2, topk = _ffn_case(rng, T, d, E, k, d_ff, 0, skew)
+    roff, rperm, _ = orc.permute(topk, E)
+    ref = orc.expert_ffn(x, rperm, roff, w1, w3, w2, act=0)
+    h = torch.empty((T * k, d_ff), device="cuda")
+    out = torch.empty((T * k, d), device="cuda")
+    ctx.expert_ffn_grouped(dev(torch, x), dev(torch, rperm), dev(torch, roff), dev(torch, w1),
+                           dev(torch, w3), dev(torch, w2), k, h, out, act=0)
+    assert_close(host(out), ref, what="expert rows")
+
+
 def test_expert_ffn_bf16_pieces_special_values(ctx, torch, orc):
     """Values that three bf16 pieces do not hold take fp32 products: infinities
     and NaN reach the outputs that they reach in fp32, the largest floats do
