@@ -1658,17 +1658,22 @@ int moe_layer_forward_noalloc(moe_ctx* ctx, const moe_layer_desc* desc,
         DeviceScope dev(ctx->device);
         FfnPlan plan = choose_ffn_plan(ctx, desc->T * desc->k, desc->d, desc->d_ff, desc->E);
         size_t need = carve_layer(nullptr, *desc, plan).bytes;
-        if (need > kNoAllocScratchBytes) {
-            // every tile whole: no partial tiles, no split partials
-            if (!plan.skinny13) plan.w13_sk = 0;
-            if (!plan.skinny2) {
-                plan.w2_sk = 0;
-                plan.splits = 1;
-            }
-            if (!plan.skinny13) plan.sk_floats = 0;
+        auto over = [&] { return need > kNoAllocScratchBytes; };
+        if (over() && plan.splits > 1) {
+            // w2's K whole: no partial row buffers
+            plan.splits = 1;
             need = carve_layer(nullptr, *desc, plan).bytes;
         }
-        if (need > kNoAllocScratchBytes)
+        if (over() && (plan.w2_sk > 0 || (plan.w13_sk > 0 && !plan.skinny13))) {
+            // ... and every tile whole: no stream-K partial tiles
+            plan.w2_sk = 0;
+            if (!plan.skinny13) {
+                plan.w13_sk = 0;
+                plan.sk_floats = 0;
+            }
+            need = carve_layer(nullptr, *desc, plan).bytes;
+        }
+        if (over())
             throw moe::InvalidArg("moe_layer_forward_noalloc: this layer needs " +
                                   std::to_string(need) + " bytes of scratch, more than the " +
                                   std::to_string(kNoAllocScratchBytes) +

@@ -332,18 +332,16 @@ int moe_layer_forward(moe_ctx* ctx, const moe_layer_desc* desc,
  * layer's workspace (logits, routing, permutation, hidden rows, w2 partials,
  * norm statistics, stream-K partial tiles) lives in a fixed 256 MiB array the
  * library holds on every GPU it runs on, until the process ends; a layer
- * needing more is rejected with MOE_ERR_INVALID.  Every layer up to 4,160
- * tokens at config 5's shape fits (3,840 behind its RMS norm), up to 3,680
- * at the reference's (1,552 behind its layer norm); some larger ones fit as
- * well, since the plan's K splits and stream-K grid change with the token
- * count (moe_ctx_reserve on a fresh context, then moe_ctx_workspace_bytes,
- * gives a layer's need).  The call allocates nothing and records no timing events.
+ * needing more is rejected with MOE_ERR_INVALID.  A layer whose plan needs
+ * more first gives up w2's K splits, then the stream-K partial tiles; its sums
+ * are then rounded in another order than moe_layer_forward's.  Every layer up
+ * to 8,700 tokens at config 5's shape fits (7,600 behind its RMS norm), up to
+ * 7,300 at the reference's (5,000 behind its layer norm).  The call allocates
+ * nothing and records no timing events.
  * Every call on one GPU shares that GPU's array, which keeps the last call's
  * contents: calls that overlap on one GPU (two streams, two threads, two
  * contexts) race and must be serialised by the caller.  Same arguments,
- * results and errors as moe_layer_forward otherwise; a layer that fits only
- * without K splits and stream-K partials runs without them, its sums then
- * rounded in another order. */
+ * results and errors as moe_layer_forward otherwise. */
 int moe_layer_forward_noalloc(moe_ctx* ctx, const moe_layer_desc* desc,
                               const moe_layer_weights* weights, const float* x,
                               float* y, int32_t* topk_idx_out, float* topk_w_out,

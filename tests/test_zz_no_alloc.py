@@ -174,6 +174,73 @@ def test_noalloc_replays_under_graph_capture(torch):
         ctx.close()
 
 
+# Layers whose plan passes the scratch: only by w2's K splits (their partial row
+# buffers taken off it fits), and also without them (the stream-K partial tiles go
+# too).  The plans are looked up, so the token count is the first that is one.
+@pytest.mark.parametrize("d,E,k,d_ff,norm,tokens,without_splits_fits", [
+    (1024, 8, 2, 2816, 0, range(5900, 8700, 100), True),
+    (4096, 4, 2, 1024, 0, range(2048, 4096, 128), True),
+    (4096, 16, 2, 448, 1, range(1000, 5000, 50), False),
+])
+def test_noalloc_plans_past_the_scratch(torch, d, E, k, d_ff, norm, tokens, without_splits_fits):
+    pkg = load_pkg()
+    cap = 256 << 20
+
+    def desc_of(T):
+        return pkg.make_desc(T, d, E, k, d_ff, act=pkg.ACT_SWIGLU, router=0, quantum=1e-3,
+                             tie_eps=2e-2, norm=pkg.NORM_LAYER if norm else pkg.NORM_NONE)
+
+    found = None
+    for T in tokens:
+        c = pkg.Context(0)
+        c.reserve(desc_of(T))
+        need, splits = c.workspace_bytes(), c.w2_splits(desc_of(T))
+        c.close()
+        whole = need - (splits - 1) * T * k * d * 4
+        if need > cap and (splits > 1 and whole <= cap - 4096 if without_splits_fits
+                           else whole > cap + 4096):
+            found = T
+            break
+    if found is None:
+        pytest.skip("no such plan on this device")
+    print(f"noalloc past the scratch: d={d} T={found} need={need} splits={splits}", flush=True)
+    rng = np.random.default_rng(d + found)
+    W = _weights(torch, rng, d, E, d_ff, norm)
+    x = _dev(torch, normal(rng, (found, d)))
+    ctx = pkg.Context(0)
+    try:
+        outs = []
+        for noalloc in (True, False):
+            y = torch.full((found, d), float("nan"), device="cuda")
+            idx = torch.full((found, k), -1, dtype=torch.int32, device="cuda")
+            w = torch.full((found, k), float("nan"), device="cuda")
+            ctx.layer_forward(desc_of(found), W, x, y, idx, w, noalloc=noalloc)
+            if noalloc:
+                assert ctx.workspace_bytes() == 0
+            outs.append((y, idx, w))
+        torch.cuda.synchronize()
+        (y1, i1, w1), (y0, i0, w0) = outs
+        assert torch.equal(i0, i1) and torch.equal(w0, w1)
+        # the same products in another order: sums of up to 4,096 columns, 1e-6 of
+        # the result each way
+        err = float((y1.double() - y0.double()).norm() / y0.double().norm())
+        assert err <= 4e-6, err
+        if without_splits_fits:
+            # only the splits went: bit for bit the stages, whose w2 has none
+            offs = torch.empty(E + 1, dtype=torch.int32, device="cuda")
+            perm = torch.empty(found * k, dtype=torch.int32, device="cuda")
+            inv = torch.empty_like(perm)
+            ctx.permute(i1, E, offs, perm, inv)
+            h = torch.empty((found * k, d_ff), device="cuda")
+            rows = torch.empty((found * k, d), device="cuda")
+            ctx.expert_ffn_grouped(x, perm, offs, W["w1"], W["w3"], W["w2"], k, h, rows)
+            y = torch.empty((found, d), device="cuda")
+            ctx.combine(rows, i1, w1, inv, y)
+            assert torch.equal(y, y1)
+    finally:
+        ctx.close()
+
+
 def test_noalloc_rejects_a_layer_beyond_the_scratch(torch):
     pkg = load_pkg()
     ctx = pkg.Context(0)
