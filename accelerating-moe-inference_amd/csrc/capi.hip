@@ -328,6 +328,16 @@ DensePlan plan_dense(moe_ctx* ctx, bool nn, bool direct, int64_t M, int64_t N, i
                                                                                      : best;
 }
 
+// Whether work on the stream is being captured in a graph.
+bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+        (void)hipGetLastError();  // (the default stream beside another one's capture)
+        return false;
+    }
+    return status == hipStreamCaptureStatusActive;
+}
+
 // C = A B (+ bias) (+ resid): resid [M, N] (may be C itself) is added after
 // the bias in the GEMM's store, or in the split reduction when K is split,
 // so C is bit-identical to the GEMM followed by moe_add.
@@ -348,7 +358,12 @@ void sgemm(moe_ctx* ctx, bool nn, const float* A, const float* B,
     const bool vec = (K % 4 == 0) && aligned16(A) && (nn || aligned16(B));
     // the direct-load kernels (every tile shape; split K): see launch_cfg
     const bool direct = vec && K % 16 == 0 && (!nn || (N % 4 == 0 && aligned16(B)));
-    const DensePlan plan = plan_dense(ctx, nn, direct, M, N, K);
+    DensePlan plan = plan_dense(ctx, nn, direct, M, N, K);
+    // A captured product whose partials the workspace does not hold runs its K
+    // whole: growing it would end the capture.
+    if (plan.splits > 1 && size_t(plan.splits) * M * N * sizeof(float) > ctx->ws_bytes &&
+        capturing(as_stream(stream)))
+        plan.splits = 1;
     const moe::GemmTile tile = moe::dense_tile(plan.tile);
     const int64_t mt = moe::ceil_div(M, tile.bm), ntl = moe::ceil_div(N, tile.bn);
     moe::require(mt * ntl * plan.splits <= INT32_MAX, "GEMM grid too large");

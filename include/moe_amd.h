@@ -127,8 +127,11 @@ typedef struct moe_layer_weights {
 int moe_ctx_create(int device, moe_ctx** out);
 int moe_ctx_destroy(moe_ctx* ctx);
 /* Grow the workspace so that moe_layer_forward(desc) allocates nothing.
- * It also covers moe_expert_ffn_grouped on the same (T, k, d, d_ff, E) and
- * the sgemm / attention calls of that size or smaller. */
+ * It also covers moe_expert_ffn_grouped on the same (T, k, d, d_ff, E).  A
+ * dense product that splits K (moe_sgemm_plan) holds its partial sums in it,
+ * splits * M * N floats, and grows it at its first call if need be; under
+ * stream capture one that would have to runs its K whole instead.  The
+ * attentions state their need below. */
 int moe_ctx_reserve(moe_ctx* ctx, const moe_layer_desc* desc);
 /* The bytes of the context's workspace as it stands (0 before any call
  * that needed one).  No reference counterpart: an introspection query for
@@ -368,7 +371,9 @@ int moe_layer_w2_splits(moe_ctx* ctx, const moe_layer_desc* desc, int32_t* split
 /* ---- the plan moe_sgemm_nn (nn != 0) or moe_sgemm_nt runs an M x N x K
  * product with on this context's device, assuming 16-byte aligned operands:
  * the tile shape id (0 128x128, 1 64x128, 2 32x128, 3 256x128, 4 the skinny
- * kernel, 5 the K-group tile) and its K splits.  No reference counterpart:
+ * kernel, 5 the K-group tile) and its K splits.  Tiles 0, 1 and 3 run on the
+ * bf16 pieces or on fp32 MFMA, whichever is modelled faster; which one is not
+ * told.  No reference counterpart:
  * an introspection query for tests and measurement tools. */
 int moe_sgemm_plan(moe_ctx* ctx, int nn, int64_t M, int64_t N, int64_t K, int32_t* tile,
                    int32_t* splits);

@@ -597,6 +597,51 @@ def test_expert_ffn_few_rows(ctx, torch, orc, T, d, E, k, d_ff, skew):
     assert_close(host(out), ref, what="expert rows")
 
 
+@pytest.mark.parametrize("layout,M,N,K", [("nt", 9, 130, 4099), ("nn", 70, 130, 4099),
+                                          ("nt", 8, 256, 4096), ("nn", 200, 256, 8192)])
+def test_sgemm_first_call_under_capture(pkg, torch, layout, M, N, K):
+    """A product whose plan splits K, captured by a context that has no workspace
+    yet: the capture holds, and every replay gives the whole-K sums, also after
+    eager calls have grown the workspace."""
+    rng = np.random.default_rng(M + K)
+    a = rng.uniform(-1, 1, (M, K)).astype(np.float32)
+    b = rng.uniform(-1, 1, (N, K)).astype(np.float32)
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    ad, bd = dev(torch, a), dev(torch, b if layout == "nt" else np.ascontiguousarray(b.T))
+    warm, fresh = pkg.Context(0), pkg.Context(0)
+    try:
+        assert fresh.sgemm_plan(M, N, K, nn=layout == "nn")["splits"] > 1
+        c = torch.zeros((M, N), device="cuda")
+
+        def product(ctx, out):
+            (ctx.sgemm_nt if layout == "nt" else ctx.sgemm_nn)(ad, bd, out)
+
+        product(warm, torch.empty_like(c))  # code objects loaded before the capture
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            product(fresh, c)
+        assert fresh.workspace_bytes() == 0
+        # fp32 sums of K products in some order: each of the K roundings at most
+        # 2^-24 of a partial sum, with random signs sqrt(K) of them
+        scale = np.sqrt(np.mean(exact ** 2))
+        first = None
+        for _ in range(3):
+            c.zero_()
+            graph.replay()
+            eager = torch.empty_like(c)
+            product(fresh, eager)
+            torch.cuda.synchronize()
+            for got in (c, eager):
+                err = np.sqrt(np.mean((host(got) - exact) ** 2)) / scale
+                assert err <= 2.0 ** -24 * np.sqrt(K)
+            first = host(c) if first is None else first
+            assert np.array_equal(host(c), first)
+    finally:
+        warm.close()
+        fresh.close()
+
+
 def test_expert_ffn_bf16_pieces_special_values(ctx, torch, orc):
     """Values that three bf16 pieces do not hold take fp32 products: infinities
     and NaN reach the outputs that they reach in fp32, the largest floats do
