@@ -141,33 +141,38 @@ constexpr int64_t kDenseSplitBytes = int64_t(512) << 20;  // cap on the partials
 // The tile and K splits of a dense product on the bf16 pieces (split.hpp) and
 // their modelled time.  A K step of r workgroups on a CU takes r times its
 // share of the matrix cores, or what one workgroup needs alone (its loads,
-// split, LDS and MFMAs in turn), from MI355X times of 16 shapes x 4 tiles x 4
-// splits: 2048^3 on 128 x 128 tiles, one per CU, 101 us; 4096^3 on 256 x 128,
-// two per CU, 660-790; 1024^3 on 64 x 128, one per CU, 35; 4096 x 1024 x 1024
-// there, two per CU, 59.  A round starts and ends in about what a 4-step
-// product (200 x 520 x 64) takes: 14, 9 and 24 us per tile.  A workgroup
-// alone takes the slower of the step times it was seen to take: they depend on
-// where the operands lie in memory (1419 x 2432 x 6720 on 128 x 128, 228
-// workgroups, 274 us in one process and 460 in the next).  With few m-tiles B comes from HBM and the steps wait
-// longer: 175 x 10816 x 7168 on 64 x 128, two per CU, 1.15 us per step.
+// split, LDS and MFMAs in turn); a round of as many as the CU holds at once
+// (the kernel's own occupancy) starts and ends in kRound.  Fitted to MI355X
+// times of 222 shapes, M 16-8,192, N 64-32,000, K 3-8,192, both layouts, ragged
+// and aligned, x 3 tiles x 4 splits: off by 11 % on average.  Of the plans within
+// 5 % of the least the one with the most splits is taken, whose shorter sums are
+// the more precise: 0.4 % slower than the best of the twelve, 11 % at worst.  With
+// 3 workgroups of 128 x 128 per CU for the 2 that their registers leave, 22 of 222
+// shapes lost more than a tenth: 3456 x 2328 x 36 31 us for 23, 5000 x 2326 x 40
+// 34.5 for 28.
 // Whole: K in whole steps of equal splits, as the fp32 tiles need it too; else
 // the splits are whole steps but for the last.  Up to 64 rows the product is
 // bound by reading B and the fp32 tiles, loading two steps ahead, are as fast
-// (64 x 14336 x 4096 76 us against 65-82); otherwise the pieces are taken where
-// their estimate is 5 % lower, the spread of the fp32 fit.
+// (64 x 14336 x 4096 76 us against 65-82).  Otherwise the pieces are taken where
+// the fp32 plan would have a 128 x 128, 64 x 128 or 256 x 128 tile (of 69 such
+// shapes they were level or faster in 68, 9 % slower in 551 x 128 x 2816), and
+// where it has the 32 x 128 one, small products that are up to 30 % faster on it,
+// if their estimate is 5 % lower, the spread of the fp32 fit.
 struct PiecesPlan {
     DensePlan plan;
     double seconds = 1e30;
 };
 
-PiecesPlan plan_pieces(moe_ctx* ctx, int64_t M, int64_t N, int64_t K, bool whole) {
+PiecesPlan plan_pieces(moe_ctx* ctx, bool nn, int64_t M, int64_t N, int64_t K, bool whole) {
     static const int env_tile = env_int("MOE_DENSE_TILE", -1);
     static const int env_splits = env_int("MOE_DENSE_SPLITS", 0);
-    static constexpr double kStep[4] = {0.70e-6, 0.42e-6, 0.0, 1.35e-6};
-    static constexpr double kAlone[4] = {1.0e-6, 0.8e-6, 0.0, 1.6e-6};
-    static constexpr double kRound[4] = {9e-6, 4.5e-6, 0.0, 16e-6};
+    static constexpr double kStep[4] = {0.584e-6, 0.415e-6, 0.0, 1.02e-6};
+    static constexpr double kAlone[4] = {0.72e-6, 0.542e-6, 0.0, 1.14e-6};
+    static constexpr double kRound[4] = {9.1e-6, 4.9e-6, 0.0, 18.9e-6};
     constexpr double kHbm = 5.0e12, kLaunch = 2e-6, kReduce = 2e-6;
-    PiecesPlan best;
+    PiecesPlan tried[3 * 5];
+    int count = 0;
+    double least = 1e30;
     for (int t : {0, 1, 3}) {
         if (env_tile >= 0 && t != env_tile) continue;
         // (its form for any K and alignment needs more registers than two
@@ -175,9 +180,8 @@ PiecesPlan plan_pieces(moe_ctx* ctx, int64_t M, int64_t N, int64_t K, bool whole
         if (t == 3 && !whole) continue;
         const moe::GemmTile g = moe::dense_tile(t);
         const int64_t mt = moe::ceil_div(M, g.bm), nt = moe::ceil_div(N, g.bn);
-        // resident per CU: 38 KB (64 x 128), 51 KB and 76 KB of LDS stages
-        const int64_t occ = t == 1 ? 4 : (t == 0 ? 3 : 2);
-        const double cold = M <= 256 ? 1.2 : 1.0;
+        int& occ = ctx->pieces_blocks_per_cu[whole ? 1 : 0][nn ? 1 : 0][t];
+        if (occ == 0) occ = moe::pieces_blocks_per_cu(t, nn, !whole);
         for (int S = 1; S <= moe::kMaxDenseSplits; S *= 2) {
             if (env_splits > 0 && S != env_splits) continue;
             const int64_t len = moe::ceil_div(moe::ceil_div(K, S), 16) * 16;
@@ -189,18 +193,24 @@ PiecesPlan plan_pieces(moe_ctx* ctx, int64_t M, int64_t N, int64_t K, bool whole
             const double steps = double(moe::ceil_div(len, 16));
             auto round_time = [&](int64_t r) {
                 if (r == 0) return 0.0;
-                return steps * cold * std::max(double(r) * kStep[t], kAlone[t]) + kRound[t];
+                return steps * std::max(double(r) * kStep[t], kAlone[t]) + kRound[t];
             };
             const double t_cu = double(per_cu / occ) * round_time(occ) + round_time(per_cu % occ);
             const double part_bytes = S > 1 ? 4.0 * S * double(M) * N : 0.0;
             const double bytes = 4.0 * (double(M) * K + double(K) * N * mt + double(M) * N);
-            double est = std::max(t_cu, (bytes + 2 * part_bytes) / kHbm) + kLaunch;
-            if (S > 1) est += kReduce + (part_bytes + 4.0 * M * N) / 4e12 + part_bytes / kHbm;
-            if (est < best.seconds) {
-                best.seconds = est;
-                best.plan = {t, S, false};
-            }
+            double est = std::max(t_cu, (bytes + 1.36 * part_bytes) / kHbm) + kLaunch;
+            if (S > 1) est += kReduce + (part_bytes + 4.0 * M * N) / 5.2e12 + part_bytes / 6e12;
+            tried[count++] = {{t, S, false}, est};
+            least = std::min(least, est);
         }
+    }
+    PiecesPlan best;
+    for (int i = 0; i < count; ++i) {
+        const PiecesPlan& p = tried[i];
+        if (p.seconds > 1.05 * least) continue;
+        if (best.seconds > 1e29 || p.plan.splits > best.plan.splits ||
+            (p.plan.splits == best.plan.splits && p.seconds < best.seconds))
+            best = p;
     }
     return best;
 }
@@ -218,7 +228,7 @@ DensePlan plan_dense(moe_ctx* ctx, bool nn, bool direct, int64_t M, int64_t N, i
         // fp32 MFMA / pieces at K = 1, 2, 3, 4: 2.5 / 3.4, 3.1 / 3.4, 3.6 / 3.3,
         // 4.0 / 3.2 e-8; largest, in 2^-24 of the products' magnitudes, 1.0 /
         // 2.5, 1.9 / 2.8, 2.5 / 2.2, 3.0 / 2.1).
-        return K > 2 && moe::pieces_fit(nn, M, N, K) ? plan_pieces(ctx, M, N, K, false).plan : best;
+        return K > 2 && moe::pieces_fit(nn, M, N, K) ? plan_pieces(ctx, nn, M, N, K, false).plan : best;
     }
     static const int env_tile = env_int("MOE_DENSE_TILE", -1);
     static const int env_splits = env_int("MOE_DENSE_SPLITS", 0);
@@ -323,9 +333,9 @@ DensePlan plan_dense(moe_ctx* ctx, bool nn, bool direct, int64_t M, int64_t N, i
         return best;
     }
     if (M <= 64) return best;
-    const PiecesPlan pieces = plan_pieces(ctx, M, N, K, true);
-    return pieces.seconds < 0.95 * best_t || (env_tile >= 0 && pieces.seconds < 1e30) ? pieces.plan
-                                                                                     : best;
+    const PiecesPlan pieces = plan_pieces(ctx, nn, M, N, K, true);
+    if (best.tile == 2 && env_tile < 0 && pieces.seconds >= 0.95 * best_t) return best;
+    return pieces.seconds < 1e30 ? pieces.plan : best;
 }
 
 // Whether work on the stream is being captured in a graph.

@@ -87,6 +87,8 @@ inline bool pieces_fit(bool nn, int64_t M, int64_t N, int64_t K) {
 GemmTile dense_tile(int tile);
 // Workgroups of dense tile shape `tile` (direct-load kernel) one CU holds at once.
 int dense_blocks_per_cu(int tile, bool nn);
+// ... of its form on the bf16 pieces (tiles 0, 1 and 3; any: for any K and alignment).
+int pieces_blocks_per_cu(int tile, bool nn, bool any);
 // K groups of a dense tile shape (1, or the K-group tiles' count).
 int dense_tile_groups(int tile);
 constexpr int kMaxDenseSplits = 16;  // split-K of a dense SGEMM (partials in the workspace)
@@ -270,6 +272,7 @@ struct moe_ctx {
     int sk_blocks_per_cu[2][5] = {};
     int sk_mode = -1;  // moe_ctx_set_stream_k: -1 planner (or MOE_SK), 0 off, 1 on
     int dense_blocks_per_cu[2][moe::kDenseTiles] = {};  // [nn][tile], lazily queried
+    int pieces_blocks_per_cu[2][2][moe::kDenseTiles] = {};  // [whole][nn][tile], lazily queried
     void* ws = nullptr;
     size_t ws_bytes = 0;
     void* scratch = nullptr;   // this device's no-alloc scratch (moe_layer_forward_noalloc)

@@ -2510,6 +2510,35 @@ int dense_blocks_per_cu(int tile, bool nn) {
 }
 
 namespace {
+template <class C>
+int pieces_occupancy(bool nn, bool any) {
+    int n = 0;
+    auto query = [&](auto kernel) {
+        hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, C::THREADS, 0),
+                  "hipOccupancyMaxActiveBlocksPerMultiprocessor");
+    };
+    if constexpr (C::BM < 256) {
+        if (any) {
+            if (nn) query(gemm_split_kernel<C, true, false, 1, EPI_BIAS, true>);
+            else query(gemm_split_kernel<C, false, false, 1, EPI_BIAS, true>);
+            return n > 0 ? n : 1;
+        }
+    }
+    if (nn) query(gemm_split_kernel<C, true, false, 1, EPI_BIAS, false>);
+    else query(gemm_split_kernel<C, false, false, 1, EPI_BIAS, false>);
+    return n > 0 ? n : 1;
+}
+}  // namespace
+
+int pieces_blocks_per_cu(int tile, bool nn, bool any) {
+    switch (tile) {
+        case 1: return pieces_occupancy<DenseMidCfg>(nn, any);
+        case 3: return pieces_occupancy<DenseTallCfg>(nn, any);
+        default: return pieces_occupancy<DenseCfg>(nn, any);
+    }
+}
+
+namespace {
 template <class C, int SCHED, int NB, int EPI>
 int grouped_occupancy(bool fp32, bool sk) {
     int n = 0;

@@ -597,6 +597,18 @@ def test_expert_ffn_few_rows(ctx, torch, orc, T, d, E, k, d_ff, skew):
     assert_close(host(out), ref, what="expert rows")
 
 
+@pytest.mark.parametrize("nn", [False, True])
+def test_sgemm_plan_of_short_products_fills_the_last_round(ctx, torch, nn):
+    """Two workgroups of 128 x 128 pieces fit a CU, so a product of few columns
+    that has a few more than 512 of them (256 CUs) would start a round for those:
+    its plan has smaller tiles."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the tile counts are for 256 CUs")
+    for M, N, K in ((3456, 2328, 36), (3727, 2326, 4), (3264, 3001, 20)):
+        assert 512 < -(-M // 128) * -(-N // 128) < 768
+        assert ctx.sgemm_plan(M, N, K, nn=nn)["tile"] == 1
+
+
 @pytest.mark.parametrize("layout,M,N,K", [("nt", 9, 130, 4099), ("nn", 70, 130, 4099),
                                           ("nt", 8, 256, 4096), ("nn", 200, 256, 8192)])
 def test_sgemm_first_call_under_capture(pkg, torch, layout, M, N, K):
