@@ -538,16 +538,21 @@ bool launch_flash_attention(const float* q, const float* k, const float* v, floa
     };
     // Four waves, two workgroups per CU, or eight waves with two stages of
     // planes, which stage half as much per wave and meet once per block but
-    // balance the causal tiles less finely (us on MI355X, fp32 MFMA / four / eight
-    // waves: head_dim 64, 512 tiles of 128 queries 54.4 / 48.2 / 52.6, 1,024 tiles
-    // 315 / 224 / 187; head_dim 128, where four waves spill 37 registers, 512 tiles
-    // 167 / 142 / 141, 1,024 tiles 684 / 501 / 378).  Up to 256 tiles of head_dim
-    // 128, at most one workgroup per CU, are bound by one wave's chain through its
-    // key blocks, which the splits lengthen: 81 / 85 / 85 and 46.6 / 51 / 49.8.
+    // balance the causal tiles less finely, and whose 256-query tiles walk blocks
+    // that a short sequence or window hides from most of their waves.  us on
+    // MI355X, fp32 MFMA / four / eight waves: head_dim 64, 512 tiles of 128 queries
+    // 54.4 / 41.2 / 52.6; 1,024 tiles and more, 2,048 keys 313 / 201 / 191, 1,396 keys
+    // 604 / 388 / 453, 100 keys 83 / 57 / 98, windows of 16 / 64 / 256 / 1,024 of 1,396
+    // keys 122 / 83 / 146, 145 / 95 / 156, 268 / 166 / 229, 547 / 360 / 393; head_dim 128
+    // (fp32 MFMA / eight waves), 512 tiles 97 / 76, 1,024 tiles 689 / 344, there with a
+    // window of 16 100 / 83.  Up to 256 tiles of head_dim 128, at most one workgroup per
+    // CU, are bound by one wave's chain through its key blocks, which the splits
+    // lengthen: 81 / 85 (four) / 85 and 46.6 / 51 / 49.8.
     const int64_t tiles = ceil_div(seq_len, 128) * batch * q_heads;
+    const int64_t keys = window > 0 && window < seq_len ? window : seq_len;
     switch (head_dim) {
         case 64:
-            if (tiles >= 1024) run(flash_attn_kernel<64, 8, true>, 8);
+            if (tiles >= 1024 && keys > 1536) run(flash_attn_kernel<64, 8, true>, 8);
             else run(flash_attn_kernel<64, 4, true>, 4);
             return true;
         case 128:

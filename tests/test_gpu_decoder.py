@@ -88,7 +88,11 @@ ATTN_CASES = [(1, 16, 1, 1, 16, None), (2, 48, 4, 2, 16, None), (2, 48, 4, 2, 16
               # at head_dim 128, 1,024 at 64): sequences off their 256-query
               # tiles, grouped heads, windows inside a key block and across them
               (4, 449, 32, 4, 128, None), (4, 400, 32, 32, 128, 21), (16, 31, 32, 2, 128, None),
-              (8, 385, 32, 4, 64, 300), (16, 129, 32, 8, 64, None)]
+              (8, 385, 32, 4, 64, 300), (16, 129, 32, 8, 64, None),
+              # head_dim 64 about the line to eight waves: 1,536 keys and 1,537, and a
+              # window of each in a longer sequence
+              (1, 1536, 86, 43, 64, None), (1, 1537, 86, 43, 64, None),
+              (1, 1800, 74, 37, 64, 1536), (1, 1800, 74, 37, 64, 1537)]
 
 
 @pytest.mark.parametrize("B,S,H,KVH,hd,window", ATTN_CASES)
