@@ -549,12 +549,13 @@ def test_expert_ffn_vs_oracle(ctx, torch, orc, request_reset_stream_k, T, d, E, 
     (161, 144, 3, 2, 144, 0), (520, 4096, 4, 2, 64, 0), (640, 64, 4, 2, 2048, 0),
 ])
 def test_expert_ffn_bf16_pieces(ctx, torch, T, d, E, k, d_ff, act):
-    """Against 64-bit sums.  Each product of pieces leaves out at most 2^-26 of
-    itself and each of the 6 K / 16 accumulations rounds once, at most 2^-23 of
-    the partial sum however the matrix unit rounds: with random signs an error
-    of about 2^-23 sqrt(6 K / 16) of the result's spread, over both products
-    at most 8 times that here (the activation's derivative, the maximum over
-    the outputs)."""
+    """Against 64-bit sums.  Each of the 6 K / 16 accumulations rounds once, at
+    most 2^-23 of the partial sum however the matrix unit rounds: with random
+    signs an error of about 2^-23 sqrt(6 K / 16) of the result's spread, over both
+    products at most 8 times that here (the activation's derivative, the maximum
+    over the outputs).  What the pieces leave out of a product, 2^-27.4 rms of it
+    and of any sign, averages away under that; test_sgemm_bf16_pieces_worst_products
+    holds it to its bound."""
     rng = np.random.default_rng(T + d + d_ff)
     x, w1, w3, w2, topk = _ffn_case(rng, T, d, E, k, d_ff, act)
     order = np.argsort(topk.ravel(), kind="stable")
@@ -655,40 +656,58 @@ def test_sgemm_first_call_under_capture(pkg, torch, layout, M, N, K):
 
 
 def test_expert_ffn_bf16_pieces_special_values(ctx, torch, orc):
-    """Values that three bf16 pieces do not hold take fp32 products: infinities
-    and NaN reach the outputs that they reach in fp32, the largest floats do
-    not overflow, and values under the smallest piece keep their precision."""
+    """Values that the bf16 pieces do not hold take fp32 products: infinities and
+    NaN reach the outputs that they reach in fp32 and no others, the largest
+    floats do not overflow where their sums do not, and every finite output is
+    the 64-bit one to the rounding of its own products' magnitudes."""
     rng = np.random.default_rng(5)
     T, d, E, k, d_ff = 300, 64, 2, 1, 160
     x, w1, w3, w2, _ = _ffn_case(rng, T, d, E, k, d_ff, 0)
     topk = (np.arange(T) % E).astype(np.int32)[:, None]
-    x[3, 5] = np.inf
-    x[40, 7] = -np.inf
+    x[3, 5] = np.inf                            # expert 1: infinities, NaN, weights of 3.4e38
+    x[41, 7] = -np.inf
     x[81, 0] = np.nan
-    x[122] = 3.4028e38 * np.sign(x[122])        # hi rounds past the largest float
-    w1[:, 17] = 1e-38 * np.sign(w1[:, 17])      # ... times tiny weights: ordinary sums
-    w3[:, 17] = 1e-38 * np.sign(w3[:, 17])
-    x[200] = 1e-37 * x[200]                     # lo under bf16's smallest denormal
     x[201] = 0.0
-    w2[0, 9] = 3.4e38 * np.sign(w2[0, 9])       # sums near and past the largest float
+    w2[1, 9] = 3.4e38 * np.sign(w2[1, 9])       # sums near and past the largest float
+    x[122] = 3.4028e38 * np.sign(x[122])        # expert 0: hi rounds past the largest float
+    w1[:, 17] = 1e-39 * np.sign(x[122])         # ... times tiny weights: ordinary sums
+    w3[:, 17] = 1e-38 * np.sign(w3[:, 17])
+    x[200] = 1e-37 * x[200]                     # below bf16's pieces, unscaled
     roff, rperm, _ = orc.permute(topk, E)
     ref = orc.expert_ffn(x, rperm, roff, w1, w3, w2, act=0)
     h = torch.empty((T * k, d_ff), device="cuda")
     out = torch.empty((T * k, d), device="cuda")
     ctx.expert_ffn_grouped(dev(torch, x), dev(torch, rperm), dev(torch, roff), dev(torch, w1),
                            dev(torch, w3), dev(torch, w2), k, h, out, act=0)
-    got = host(out)
+    got, hid = host(out), host(h)
     assert np.array_equal(np.isfinite(got), np.isfinite(ref))
-    tiny = np.flatnonzero(rperm == 200)
-    assert np.all(got[np.flatnonzero(rperm == 201)] == 0)
-    ok = np.isfinite(ref).all(axis=1)
-    for r in np.flatnonzero(ok):                # each row to its own scale
-        scale = np.max(np.abs(ref[r]))
-        assert np.max(np.abs(got[r] - ref[r])) <= 1e-4 * scale + 1e-38, r
-    # x = 1e-37 N(0, 1) against weights of 0.02: the gate and up sums, about
-    # 2e-38, in 64 bits
-    hg = host(h)[tiny[0]]
-    assert np.all(np.isfinite(hg))
+    assert np.all(got[rperm == 201] == 0)
+    # 64-bit results and what their own roundings may leave: every product 2^-24, what the
+    # pieces leave out of it 2^-24, each of 6 K / 16 additions 2^-23; the activation's few
+    # roundings 2^-21 of the hidden value, which the gate moves by at most 1.1 per unit
+    f8 = lambda t: t.astype(np.float64)
+    with np.errstate(all="ignore"):
+        for e in range(E):
+            rows = slice(roff[e], roff[e + 1])
+            xe = f8(x[rperm[rows]])
+            g, u = xe @ f8(w1[e]).T, xe @ f8(w3[e]).T
+            act = g / (1 + np.exp(-g))
+            mag = lambda w: np.abs(xe) @ np.abs(f8(w[e])).T
+            unit = lambda K: (6 * K / 16 + 2) * 2.0 ** -23
+            dh = (unit(d) * (1.1 * mag(w1) * np.abs(u) + np.abs(act) * mag(w3))
+                  + 2.0 ** -21 * np.abs(act * u) + 2.0 ** -126)
+            want_h = act * u
+            ok = np.isfinite(want_h) & (np.abs(want_h) < 3.3e38)
+            assert np.all(np.abs(hid[rows] - want_h)[ok] <= dh[ok]), e
+            aw2 = np.abs(f8(w2[e])).T
+            want = want_h @ f8(w2[e]).T
+            bound = dh @ aw2 + unit(d_ff) * (np.abs(want_h) @ aw2) + d_ff * 2.0 ** -149
+            ok = np.isfinite(ref[rows])
+            assert ok.sum() > 0.9 * ok.size * (1 if e == 0 else 0.9)
+            assert np.all(np.abs(got[rows] - want)[ok] <= bound[ok]), e
+    # the largest floats times tiny weights: a finite hidden value among infinities
+    row = int(np.flatnonzero(rperm == 122)[0])
+    assert np.isfinite(hid[row, 17]) and hid[row, 17] != 0 and not np.isfinite(hid[row]).all()
 
 
 def test_expert_ffn_bf16_pieces_tiny_rows(ctx, torch):
@@ -750,6 +769,29 @@ def test_sgemm_bf16_pieces(ctx, torch, layout, M, N, K, offset, bias):
     err = np.sqrt(np.mean((host(c) - ref) ** 2)) / max(scale, np.sqrt(np.mean(ref ** 2)))
     assert err <= 4 * 2.0 ** -23 * max(1.0, np.sqrt(6 * K / 16))
     assert bool((out[M * N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("K", [3, 15, 100, 1000, 1024])
+def test_sgemm_bf16_pieces_worst_products(ctx, torch, layout, K):
+    """Operands of one sign whose middle and low pieces are the largest, so that
+    every product loses as much as the pieces can leave out, 2^-24 of it, in one
+    direction; beside it the 6 K / 16 additions (a step of 16 columns is six)
+    round by at most 2^-23 of the sum each."""
+    M, N = 300, 200
+    worst = np.float32(1 + 2.0 ** -8 - 2.0 ** -17 - 2.0 ** -23)
+    rng = np.random.default_rng(K)
+    a = worst * np.exp2(rng.integers(-3, 4, (M, 1))).astype(np.float32) * np.ones((M, K), np.float32)
+    b = worst * np.exp2(rng.integers(-3, 4, (N, 1))).astype(np.float32) * np.ones((N, K), np.float32)
+    c = torch.empty((M, N), device="cuda")
+    if layout == "nt":
+        ctx.sgemm_nt(dev(torch, a), dev(torch, b), c)
+    else:
+        ctx.sgemm_nn(dev(torch, a), dev(torch, np.ascontiguousarray(b.T)), c)
+    exact = a.astype(np.float64) @ b.astype(np.float64).T
+    steps = -(-K // 16)
+    rel = np.abs(host(c) - exact) / exact
+    assert np.max(rel) <= 1.001 * 2.0 ** -24 + 6 * steps * 2.0 ** -23
 
 
 @pytest.mark.parametrize("layout,N,K", [("nt", 130, 64), ("nt", 129, 70), ("nn", 132, 64),
