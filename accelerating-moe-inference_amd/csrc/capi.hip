@@ -145,8 +145,9 @@ constexpr int64_t kDenseSplitBytes = int64_t(512) << 20;  // cap on the partials
 // (the kernel's own occupancy) starts and ends in kRound.  Fitted to MI355X
 // times of 222 shapes, M 16-8,192, N 64-32,000, K 3-8,192, both layouts, ragged
 // and aligned, x 3 tiles x 4 splits: off by 11 % on average.  Of the plans within
-// 5 % of the least the one with the most splits is taken, whose shorter sums are
-// the more precise: 0.4 % slower than the best of the twelve, 11 % at worst.  With
+// 5 % of the least whose partial sums are at most 16 MB the one with the most
+// splits is taken, whose shorter sums are the more precise: 0.4 % slower than the
+// best of the twelve, 11 % at worst; 90 larger shapes 0.8 %, 7 % at worst.  With
 // 3 workgroups of 128 x 128 per CU for the 2 that their registers leave, 22 of 222
 // shapes lost more than a tenth: 3456 x 2328 x 36 31 us for 23, 5000 x 2326 x 40
 // 34.5 for 28.
@@ -207,7 +208,8 @@ PiecesPlan plan_pieces(moe_ctx* ctx, bool nn, int64_t M, int64_t N, int64_t K, b
     PiecesPlan best;
     for (int i = 0; i < count; ++i) {
         const PiecesPlan& p = tried[i];
-        if (p.seconds > 1.05 * least) continue;
+        const bool small = 4.0 * p.plan.splits * double(M) * N <= 16e6;
+        if (p.seconds > (small ? 1.05 : 1.0) * least) continue;
         if (best.seconds > 1e29 || p.plan.splits > best.plan.splits ||
             (p.plan.splits == best.plan.splits && p.seconds < best.seconds))
             best = p;
@@ -525,7 +527,9 @@ int64_t expected_m_tiles(int64_t pairs, int64_t E, int bm) {
 // for one tile per workgroup.
 //
 // The bf16 pieces do the same work in half the time, so reading a tile's
-// operands alone, out of step with the tiles that share them, costs them more:
+// operands alone, out of step with the tiles that share them, costs them more (and
+// the looped kernels of the 256 x 64 w1/w3 and the 128 x 256 w2 spill 6 or 7
+// registers):
 // w1/w3 run stream-K only while the tiles fill at most 0.7 of the slots (us,
 // one tile per workgroup / stream-K: the reference's layer at 256 / 1,024 /
 // 4,096 tokens, fill 0.1 / 0.2 / 0.5, 387 / 405 / 548 against 120 / 170 / 454;
