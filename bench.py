@@ -18,7 +18,8 @@ experts top-2, SwiGLU d_ff 14336, weights N(0, 0.02), inputs N(0, 1),
 softmax over the selected logits.
 
 The default run prints ONE JSON line: config 3's tokens/s, the roofline of
-its dominant kernel (the grouped w1/w3 SwiGLU GEMM, fp32 MFMA bound)
+its dominant kernel (the grouped w1/w3 SwiGLU GEMM, bound by the matrix
+cores: six bf16 products per fp32 one, or fp32 MFMA where experts hold few rows)
 measured with HIP events on the stream the kernels run on, and the CPU path
 (the oracle restatement of the reference's PhiMoE::forward, built for this
 host with -march=native, on every core this process is given) timed on a
@@ -27,7 +28,8 @@ the baseline measured the same way in the same run, each with its roofline
 and its CPU leg: config 1 (GPU and the whole CPU layer), config 2's eight NN
 SGEMM shapes, config 4, config 5's MoE FFN, the reference's own layer shape,
 config 5's whole decoder prefill, and the drop-in PhiTinyMoEModel::generate
-on the reference's model shape.
+on the reference's model shape.  The line holds each one's main figures;
+--details FILE writes everything measured.
 """
 from __future__ import annotations
 
@@ -44,6 +46,8 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 METRIC = "MoE layer tokens/sec + expert-GEMM TFLOP/s (% fp32 MFMA peak), 1 MI355X"
 FP32_MFMA_PEAK_TFLOPS = 157.3
+# fp32 products as six products of bf16 pieces: a sixth of the dense bf16 peak
+PIECES_PEAK_TFLOPS = 2500.0 / 6
 HBM_PEAK_GBS = 8000.0
 NORM_EPS = 1e-5
 SPINUP_S = 1.0
@@ -358,6 +362,11 @@ def load_traffic(name, key="expert_w13_swiglu_bytes_per_launch"):
         return json.load(f).get(key)
 
 
+def matrix_peak(pieces):
+    """The matrix cores' fp32 peak, TFLOP/s: on the bf16 pieces or fp32 MFMA."""
+    return PIECES_PEAK_TFLOPS if pieces else FP32_MFMA_PEAK_TFLOPS
+
+
 def build_layer(pkg, cfg, T, block, dev):
     """Seeded inputs, weights, outputs and the descriptor of one layer shape."""
     import torch
@@ -460,6 +469,8 @@ def layer_entry(pkg, name, dev, warmup, steps, cpu_seconds, block=False, tokens=
     w13_ms, w2_ms = avg[w13_name], avg["expert_w2"]
     w13_tflops = flops_w13 / (w13_ms * 1e-3) / 1e12
     expert_tflops = (flops_w13 + flops_w2) / ((w13_ms + w2_ms) * 1e-3) / 1e12
+    # above 32 rows per expert no launch is on the fp32 MFMA kernels for few rows
+    peak = matrix_peak(pairs > 32 * E and d % 16 == 0 and d_ff % 16 == 0)
     entry = {
         "workload": cfg["workload"],
         "config": {"workload": cfg["workload"], "tokens": T, "d_model": d, "experts": E,
@@ -482,9 +493,9 @@ def layer_entry(pkg, name, dev, warmup, steps, cpu_seconds, block=False, tokens=
             "kernel": w13_name,
             "bound": "mfma",
             "achieved": w13_tflops,
-            "peak": FP32_MFMA_PEAK_TFLOPS,
+            "peak": peak,
             "unit": "TFLOP/s",
-            "frac": w13_tflops / FP32_MFMA_PEAK_TFLOPS,
+            "frac": w13_tflops / peak,
             "traffic": (load_traffic(name, f"{w13_name}_bytes_per_launch")
                         if (tokens is None and not block) else None),
             "flops_per_launch": flops_w13,
@@ -544,15 +555,17 @@ def sgemm_time(ctx, fn, a, b, c, warmup, steps, spin_s):
     return e0.elapsed_time(e1) * 1e-3 / steps, wall
 
 
-def sgemm_roofline(M, N, K, t):
+def sgemm_roofline(M, N, K, t, plan):
     flops = 2.0 * M * N * K
     nbytes = 4.0 * (M * K + K * N + M * N)
-    t_flop = flops / (FP32_MFMA_PEAK_TFLOPS * 1e12)
+    # aligned products of more than 64 rows on these tiles run on the pieces
+    peak = matrix_peak(M > 64 and plan["tile"] in (0, 1, 3))
+    t_flop = flops / (peak * 1e12)
     t_byte = nbytes / (HBM_PEAK_GBS * 1e9)
     hbm = t_byte > t_flop
     return {"bound": "hbm" if hbm else "mfma",
             "achieved": (nbytes / t / 1e9) if hbm else flops / t / 1e12,
-            "peak": HBM_PEAK_GBS if hbm else FP32_MFMA_PEAK_TFLOPS,
+            "peak": HBM_PEAK_GBS if hbm else peak,
             "unit": "GB/s" if hbm else "TFLOP/s",
             "frac": max(t_flop, t_byte) / t}
 
@@ -586,7 +599,7 @@ def sgemm_entries(pkg, warmup, steps, cpu_seconds):
         e = {"layout": "nn", "M": M, "N": N, "K": K, "ms_per_call": t * 1e3, "wall_ms": wall * 1e3,
              "tflops": flops / t / 1e12,
              "frac_fp32_mfma_peak": flops / t / 1e12 / FP32_MFMA_PEAK_TFLOPS}
-        roof = sgemm_roofline(M, N, K, t)
+        roof = sgemm_roofline(M, N, K, t, ctx.sgemm_plan(M, N, K, nn=True))
         e["frac_of_roofline_time"] = roof["frac"]
         e["roofline"] = dict(roof, traffic=traffic.get(f"nn {M}x{N}x{K}"))
         if oracle is not None:
@@ -632,12 +645,13 @@ def sgemm_sweep(args):
                                  SPINUP_S if first else SPINUP_S / 5)
             first = False
             flops = 2.0 * M * N * K
+            plan = ctx.sgemm_plan(M, N, K, nn=layout == "nn")
             print(json.dumps({"workload": "sgemm", "layout": layout, "M": M, "N": N, "K": K,
-                              "plan": ctx.sgemm_plan(M, N, K, nn=layout == "nn"),
+                              "plan": plan,
                               "ms_per_call": t * 1e3, "wall_ms": wall * 1e3,
                               "tflops": flops / t / 1e12,
                               "frac_fp32_mfma_peak": flops / t / 1e12 / FP32_MFMA_PEAK_TFLOPS,
-                              "frac_of_roofline_time": sgemm_roofline(M, N, K, t)["frac"]}),
+                              "frac_of_roofline_time": sgemm_roofline(M, N, K, t, plan)["frac"]}),
                   flush=True)
             del a, b, c
     ctx.close()
@@ -798,9 +812,9 @@ def decoder_entry(pkg, warmup, steps, cpu_seconds, graph=True):
             "kernel": "expert_w13_swiglu",
             "bound": "mfma",
             "achieved": w13_tflops,
-            "peak": FP32_MFMA_PEAK_TFLOPS,
+            "peak": PIECES_PEAK_TFLOPS,
             "unit": "TFLOP/s",
-            "frac": w13_tflops / FP32_MFMA_PEAK_TFLOPS,
+            "frac": w13_tflops / PIECES_PEAK_TFLOPS,
             "traffic": load_traffic("c5"),
             "flops_per_step": flops_w13,
             "launches_per_step": cfg.layers,
@@ -1107,7 +1121,7 @@ def model_entry(warmup, steps, cpu_seconds):
                    "experts": PHI["E"], "top_k": 2, "d_ff": PHI["d_ff"], "vocab": PHI["vocab"],
                    "router": "quantised top-2, weights 1/2 (PhiMoE::route)"},
         "model_tflops": flops / (ms.value * 1e-3) / 1e12,
-        "model_frac_fp32_mfma_peak": flops / (ms.value * 1e-3) / 1e12 / FP32_MFMA_PEAK_TFLOPS,
+        "model_frac_pieces_peak": flops / (ms.value * 1e-3) / 1e12 / PIECES_PEAK_TFLOPS,
         "flops_note": ("projections, experts and lm_head over the prefix-trie rows; attention "
                        "(under 1 % of the FLOPs) left out; host-to-device token copy and "
                        "device-to-host logits copy inside the time"),
@@ -1160,6 +1174,37 @@ def other_configs(pkg, dev, warmup, steps):
     return out
 
 
+def brief(e):
+    """An entry's main figures, five digits each: what fits a line beside the
+    other configurations'."""
+    def digits(v):
+        if isinstance(v, float):
+            return float(f"{v:.5g}")
+        return {k: digits(x) for k, x in v.items()} if isinstance(v, dict) else v
+
+    if isinstance(e, list):
+        return [brief(x) for x in e]
+    if "error" in e:
+        return e
+    keep = ("M", "N", "K", "value", "unit", "ms_per_step", "ms_per_call", "tflops",
+            "expert_gemm_tflops", "model_tflops")
+    out = {k: e[k] for k in keep if k in e}
+    if e.get("config"):
+        out["workload"] = e["config"]["workload"]
+    roof = e.get("roofline")
+    if roof:
+        out["roofline"] = {k: roof[k] for k in ("kernel", "bound", "achieved", "peak", "frac")
+                           if k in roof}
+    cpu, parity = e.get("cpu_baseline"), e.get("cpu_sample_parity")
+    if cpu:
+        out["cpu"] = {k: cpu[k] for k in ("value", "unit") if k in cpu}
+    if parity:
+        out["parity"] = {k: parity[k] for k in ("routing_bit_exact", "max_rel_err",
+                                                "logits_max_rel_err", "within_1e-4")
+                         if k in parity}
+    return digits(out)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1186,6 +1231,8 @@ def main():
     ap.add_argument("--dropin", action="store_true",
                     help="the C++ drop-in PhiMoE::forward at the reference's layer shape, host "
                          "tensors in and out (PCIe-inclusive)")
+    ap.add_argument("--details", metavar="FILE", default=None,
+                    help="write every measured figure there as JSON (the line holds the main ones)")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU: --gpus {args.gpus} is not supported "
@@ -1233,6 +1280,13 @@ def main():
     out.update(e)
     if args.config == "c3" and args.tokens is None and not args.block and not args.no_extra:
         out["configs"] = other_configs(pkg, dev, args.warmup, args.steps)
+    if args.details is not None:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    if "configs" in out:
+        out["configs"] = {name: brief(e) for name, e in out["configs"].items()}
+    for name in ("hbm_kernels", "expert_rows", "spinup", "timing"):  # --details only
+        out.pop(name)
     print(json.dumps(out))
 
 
