@@ -1,6 +1,7 @@
-// fp32 GEMM engine for gfx950 on the matrix cores: v_mfma_f32_32x32x2_f32,
-// and, for the expert tiles, v_mfma_f32_32x32x16_bf16 over three exact bf16
-// pieces of every fp32 value (split.hpp).
+// fp32 GEMM engine for gfx950 on the matrix cores: v_mfma_f32_32x32x16_bf16
+// over three exact bf16 pieces of every fp32 value (split.hpp) for the expert
+// tiles and the dense products of more than 64 rows, v_mfma_f32_32x32x2_f32 for
+// few rows, small products and what the pieces do not hold.
 //
 // One kernel template serves every contraction of the MoE path:
 //   dense NT  C = A B^T (+bias)       tensor_ops::matmul_transposed / Linear
@@ -1369,12 +1370,12 @@ __device__ __forceinline__ void direct_tile(const GemmArgs& p, int mt, int nt, i
 // 15.6 ms for 14.4, and a tenth of zero rows cost 5-11 % more.)
 //
 // Bound: power.  The bare MFMA loop holds about 1,750 TFLOP/s of bf16 on this
-// card at 1.7 GHz; in these tiles the matrix pipe is busy 64-74 % of the cycles
-// at 1.5 GHz.  Measured on MI355X, ms per launch and fp32 TFLOP/s, on
-// v_mfma_f32_32x32x2_f32 -> here: config 3 w1/w3 13.7 (140) -> 10.3 (187), w2
-// 6.9 (139) -> 4.9 (197); config 4 w1/w3 10.9 (138) -> 7.3 (208), w2 5.5 (138)
-// -> 3.6 (209); the reference's layer w1/w3 1.75 (131) -> 1.31 (175), w2 0.91
-// (126) -> 0.57 (201).  256 x 256 tiles of 8 waves, which load and split a
+// card at 1.7 GHz; in these tiles the matrix pipe is busy 73-83 % of the cycles
+// (w1/w3; w2 68-80 %).  Measured on MI355X, ms per launch and fp32 TFLOP/s, on
+// v_mfma_f32_32x32x2_f32 -> here: config 3 w1/w3 13.7 (140) -> 9.4 (205), w2 6.9
+// (139) -> 4.7 (206); config 4 w1/w3 10.9 (138) -> 7.2 (210), w2 5.5 (138) -> 3.7
+// (206); the reference's layer w1/w3 1.75 (131) -> 1.21 (190), w2 0.91 (126) ->
+// 0.61 (189).  256 x 256 tiles of 8 waves, which load and split a
 // third less per product, were no faster (config 3 12.2 and 5.2, config 4 7.8
 // and 3.7): one workgroup per CU stands still at its barriers.
 template <int ROWS>

@@ -507,9 +507,11 @@ void launch(const float* x, const float* w, const float* b, int64_t rows, int64_
     // Wide rows that one round of resident workgroups holds stay there too:
     // every chain runs at once, x is read once and y needs no pass of its own.
     // Measured on MI355X, us, ring and apply against resident: d = 4096 at 7 /
-    // 512 / 2,048 rows (one round) 55 / 57 / 66 against 37 / 46 / 54, at 4,096
-    // and 15,583 rows (two and eight) 80 / 191 against 99 / 379; d = 2048 at 7 /
-    // 4,096 rows (one) 30 / 42 against 20 / 35, at 8,192 (two) 55 against 68.
+    // 1,024 / 2,048 rows (one round) 55 / 57 / 66 against 36 / 46 / 49; d = 2048 at
+    // 7 / 4,096 rows (one) 30 / 42 against 19 / 31; and, resident rows dealt in
+    // chunks of 1,024 columns (2-12 % slower at these widths), d = 4096 at 4,096 and
+    // 15,583 rows (two and eight) 80 / 191 against 99 / 379, d = 2048 at 8,192 (two)
+    // 55 against 68.
     const int64_t round = hs <= kResidentFloats
                               ? 2 * static_cast<int64_t>(cus > 0 ? cus : 1) * (kResidentFloats / hs)
                               : 0;
