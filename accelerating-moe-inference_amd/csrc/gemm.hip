@@ -1557,16 +1557,20 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
                                                           boff[(i - CA) % CB], k_bytes, 0);
         }
     };
-    // the chunk's columns of the step at ktail, zeros past K
+    // the chunk's columns of the step at ktail, zeros past K.  Past the ends the
+    // loads repeat the last column and the zeros are chosen after: loads under a
+    // condition wait for each other (3727 x 2326 x 4 20 us for 17).
     auto load_tail = [&](int i) {
         auto& st = stages[0];
         if (NN && i >= CA) {
+            const int64_t n = n0 + 2 * pair, c0 = n < N ? n : N - 1, c1 = n + 1 < N ? n + 1 : N - 1;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int64_t k = ktail + 4 * kq + j, n = n0 + 2 * pair;
-                const float* row = B[0] + k * p.ldb;
-                st[CA][j] = __float_as_uint(k < K && n < N ? row[n] : 0.0f);
-                st[CA + (NN ? 1 : 0)][j] = __float_as_uint(k < K && n + 1 < N ? row[n + 1] : 0.0f);
+                const int64_t k = ktail + 4 * kq + j;
+                const float* row = B[0] + (k < K ? k : K - 1) * p.ldb;
+                const float v0 = row[c0], v1 = row[c1];
+                st[CA][j] = __float_as_uint(k < K && n < N ? v0 : 0.0f);
+                st[CA + (NN ? 1 : 0)][j] = __float_as_uint(k < K && n + 1 < N ? v1 : 0.0f);
             }
             return;
         }
@@ -1575,7 +1579,8 @@ __device__ __forceinline__ void split_tile(const GemmArgs& p, int mt, int nt, in
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int64_t k = ktail + (c & 3) * 4 + j;
-            st[i][j] = __float_as_uint(k < K ? row[k] : 0.0f);
+            const float v = row[k < K ? k : K - 1];
+            st[i][j] = __float_as_uint(k < K ? v : 0.0f);
         }
     };
     // the pieces of four consecutive k of an operand's row, to `at` + 8 bytes per piece plane
